@@ -159,6 +159,28 @@ template <typename T>
 void kn_chain_init(const KnChainWork<T> &w, int l);
 void zero_u64(unsigned long long *p, int n);
 
+// The whole KN loop in one launch (small l and Nl, kn_loop.hip).  run() iterates from X = [I; 0]
+// (resume: from the state [X | B | Bg | G], Nl x l blocks, in `state`) on the symmetric M until
+// ||C - I||_F <= tol, until itmax iterations are done in all (it0 before this call), or for maxit
+// iterations, and leaves the state there.  scal (device-visible, e.g. a pinned slot): [0]
+// ||C - I||_F, [1] iterations done in all, [2] rho, [3] status: 0 converged or itmax reached (only
+// X is left); 1 rho out of reach of the series and of Newton-Schulz (or mode 1) in the iteration
+// after those done: the state with its G is left for the caller's eigendecomposition; 2 a grid
+// barrier timed out; 3 maxit iterations done.
+template <typename T>
+bool kn_loop_fits(i64 l, i64 Nl);
+int kn_loop_mode();  // ISVD_KN_LOOP=0: never (a test hook)
+template <typename T>
+struct KnLoop {
+  i64 l, Nl;
+  int blocks;
+  DBuf<T> buf;
+  DBuf<unsigned long long> bar;
+  KnLoop(i64 l, i64 Nl);
+  void run(const T *M, T ninv, T *state, bool resume, i64 it0, i64 itmax, i64 maxit, double tol,
+           int mode, double *scal);
+};
+
 
 // In-place inverse (Gauss-Jordan, partial pivoting), n <= 128; *info_dev = 0 or the 1-based
 // index of a zero pivot.

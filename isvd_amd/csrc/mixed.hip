@@ -97,6 +97,13 @@ void stage_integrate_kn_b(const Dims &d, const KnArgs &args, const float *yst, i
                           float *qt, i64 ldqt, i64 *iter, double *err) {
   const i64 l = d.l, Nl = d.Nl;
   DBuf<float> x32(Nl * l);
+  if (kn_loop_takes<float>(l, Nl)) {  // one launch, products with M itself in FP32
+    DBuf<float> m32(Nl * Nl);
+    gram_split(d, yst, ldyst, m32.get());
+    integrate_kn_coords<float>(d, args, m32.get(), x32.get(), iter, err, nullptr);
+    gemm<float>('T', 'N', l, d.m, Nl, 1.f, x32.get(), Nl, yst, ldyst, 0.f, qt, ldqt);
+    return;
+  }
   // M as its two BF16 terms: the FP32 loop iterates with M'' = Mh + Ml and takes its products
   // with M'' on the BF16 matrix cores
   DBuf<uint16_t> S(2 * Nl * Nl), bop(2 * Nl * 3 * l);

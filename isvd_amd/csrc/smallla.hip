@@ -7,6 +7,7 @@
 //    (I/2 + (I/4 - Z)^{1/2})^{1/2} by a Taylor series or coupled Newton-Schulz square roots);
 //  - inv_small: Gauss-Jordan inverse with partial pivoting, matrix held in LDS.
 #include "dpp.hpp"
+#include "kn_common.hpp"
 #include "la.hpp"
 
 #include <cmath>
@@ -14,26 +15,7 @@
 
 namespace isvd {
 
-typedef double d4s __attribute__((ext_vector_type(4)));
-typedef float f4s __attribute__((ext_vector_type(4)));
-
 namespace {
-
-template <typename T> struct SM;
-template <> struct SM<double> {
-  using acc = d4s;
-  static __device__ __forceinline__ acc mfma(double a, double b, acc c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int lane, int g) { return (lane >> 4) + 4 * g; }
-};
-template <> struct SM<float> {
-  using acc = f4s;
-  static __device__ __forceinline__ acc mfma(float a, float b, acc c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int lane, int g) { return 4 * (lane >> 4) + g; }
-};
 
 constexpr int kSmallMaxK = 128;
 
@@ -248,20 +230,6 @@ namespace {
 // ---------------------------------------------------------------------------------------------
 constexpr int kChainWaves = 8;
 constexpr int kChainThreads = 64 * kChainWaves;
-constexpr unsigned kChainSpinLimit = 1u << 22;  // ~4 s of polling
-constexpr int kSeriesBlocks = 8;                // Paterson-Stockmeyer blocks of 4 powers
-constexpr int kSeriesTerms = 4 * kSeriesBlocks + 1;
-
-enum { kBarCount = 0, kBarAbort = 1 };
-
-template <typename T>
-__device__ __forceinline__ T cld(const T *p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <typename T>
-__device__ __forceinline__ void cst(T *p, T v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 
 // extra work of a product's epilogue, per output entry v at (r, c) (bit flags)
 enum ChainEpi {
@@ -347,12 +315,6 @@ __device__ T chain_sum(const T *v, int n, T *sh) {
   const T r = *sh;
   __syncthreads();
   return r;
-}
-
-// sum_j c[j] Z^j (j < 4) at entry e, Z^0 = I
-template <typename T>
-__device__ __forceinline__ T block_at(const T *c, T dl, T z, T z2, T z3) {
-  return c[0] * dl + c[1] * z + c[2] * z2 + c[3] * z3;
 }
 
 // One round over this workgroup's two tiles (2 wg, 2 wg + 1): product p0 and, with Dual, p1.
@@ -488,34 +450,6 @@ template <typename T>
 __device__ __forceinline__ void round2(const ChainArgs<T> &a, const ChainProd<T> &p0,
                                        const ChainProd<T> &p1, typename SM<T>::acc (*red)[64]) {
   chain_round<T, true>(a, p0, p1, red);
-}
-
-// Paterson-Stockmeyer blocks (of 4 powers) needed for the Taylor series of f and g to reach
-// a quarter of the unit roundoff for 4 ||Z||_2 <= rho; 0 when more than kSeriesBlocks would be.
-// The tail past degree 4t - 1 is bounded by the tabulated terms up to kSeriesTerms - 1 plus the
-// last one again (for rho < 1/2 the terms decay at least geometrically with ratio < 1/2).
-template <typename T>
-__device__ int series_blocks(const T *coef, double rho) {
-  const double eps = (sizeof(T) == 8) ? 0x1p-53 : 0x1p-24;
-  if (!(rho < 0.5)) return 0;
-  const double x = rho / 4.0;
-  double tf[kSeriesTerms], tg[kSeriesTerms];
-  double xp = 1.0;
-  for (int k = 0; k < kSeriesTerms; ++k) {
-    tf[k] = fabs((double)coef[k]) * xp;
-    tg[k] = fabs((double)coef[kSeriesTerms + k]) * xp;
-    xp *= x;
-  }
-  // tails from degree k on (suffix sums); the smallest t whose tail from 4t on is small enough
-  double rf = tf[kSeriesTerms - 1], rg = tg[kSeriesTerms - 1];
-  int best = 0;
-  for (int k = kSeriesTerms - 1; k >= 4; --k) {
-    rf += tf[k];
-    rg += tg[k];
-    if ((k & 3) == 0 && k / 4 <= kSeriesBlocks && rf <= 0.25 * eps && rg <= 0.25 * eps)
-      best = k / 4;
-  }
-  return best;
 }
 
 template <typename T>
@@ -795,7 +729,7 @@ void kn_chain(int l, T ninv, const T *parts, int nparts, T *DDg, const KnChainWo
 }
 
 template <typename T>
-void kn_chain_init(const KnChainWork<T> &w, int l) {
+const T *series_table() {
   static const std::vector<T> table = [] {
     long double cf[kSeriesTerms], cg[kSeriesTerms];
     series_coefficients(cf, cg, kSeriesTerms);
@@ -806,9 +740,14 @@ void kn_chain_init(const KnChainWork<T> &w, int l) {
     }
     return v;
   }();
+  return table.data();
+}
+
+template <typename T>
+void kn_chain_init(const KnChainWork<T> &w, int l) {
   const i64 ll = (i64)l * l;
-  HIP_CHECK(hipMemcpyAsync(w.buf + 9 * ll + kKnChainPart, table.data(), sizeof(T) * table.size(),
-                           hipMemcpyHostToDevice, ctx().stream));
+  HIP_CHECK(hipMemcpyAsync(w.buf + 9 * ll + kKnChainPart, series_table<T>(),
+                           sizeof(T) * 2 * kSeriesTerms, hipMemcpyHostToDevice, ctx().stream));
   zero_u64(w.bar, kKnChainBarWords);
 }
 
@@ -829,6 +768,7 @@ void inv_small(i64 n, T *A, i64 lda, int *info_dev) {
                               T *, i64, T);                                                    \
   template void inv_small<T>(i64, T *, i64, int *);                                           \
   template void kn_chain<T>(int, T, const T *, int, T *, const KnChainWork<T> &, T *, T *, int); \
+  template const T *series_table<T>();                                                        \
   template void kn_chain_init<T>(const KnChainWork<T> &, int);
 INST(double)
 INST(float)

@@ -352,6 +352,97 @@ int kn_mode() {
   return 0;
 }
 
+// Whether the KN loop runs as one launch: wherever it fits (it was the faster one at every size
+// measured; the figures are in kn_loop.hip).
+template <typename T>
+bool kn_loop_takes(i64 l, i64 Nl) {
+  return kn_loop_mode() && kn_mode() != 1 && kn_loop_fits<T>(l, Nl);
+}
+template bool kn_loop_takes<double>(i64, i64);
+template bool kn_loop_takes<float>(i64, i64);
+
+// The l x l part of one iteration by the eigendecomposition of Z, from the Gram partials:
+// C = V diag(s) V^T, s = sqrt(1/2 + sqrt(1/4 - eig(Z))), scal[0] = ||s - 1||_2, W3 as kn_chain
+// leaves it.
+template <typename T>
+void kn_eig_w3(i64 l, T ninv, const T *parts, int nparts, T *ddg, const KnChainWork<T> &chain,
+               T *w3, T *scal) {
+  const i64 ll = l * l;
+  DBuf<T> w(l), zv(ll), zs(ll), zi(ll), c(ll), cinv(ll);
+  kn_chain<T>((int)l, ninv, parts, nparts, ddg, chain, w3, scal, 1);
+  syev_small<T>(l, chain.Z(), l, w.get(), zv.get(), l);
+  hipLaunchKernelGGL(kn_scalars_kernel<T>, dim3(1), dim3(256), 0, ctx().stream, (int)l,
+                     (const T *)w.get(), (const T *)zv.get(), zs.get(), zi.get(), scal);
+  LAUNCH_CHECK();
+  small_gemm<T>('N', 'T', l, l, l, T(1), zs.get(), l, zs.get(), l, T(0), c.get(), l);
+  small_gemm<T>('N', 'T', l, l, l, T(1), zi.get(), l, zi.get(), l, T(0), cinv.get(), l);
+  hipLaunchKernelGGL(sym_from_upper_kernel<T>, dim3(grid_for(ll)), dim3(256), 0, ctx().stream,
+                     (int)l, cinv.get(), l);
+  LAUNCH_CHECK();
+  // F [in C] := C - D inv(C)  (:218)
+  small_gemm<T>('N', 'N', l, l, l, T(-1), ddg, l, cinv.get(), l, T(1), c.get(), l);
+  hipLaunchKernelGGL(kn_assemble_kernel<T>, dim3(grid_for(ll)), dim3(256), 0, ctx().stream,
+                     (int)l, (const T *)c.get(), (const T *)cinv.get(), ninv, w3);
+  LAUNCH_CHECK();
+}
+
+// The KN iteration for small l: the whole loop in one launch (KnLoop); the host enters again only
+// after an iteration that needs the eigendecomposition of Z (or kLoopChunk iterations).
+template <typename T>
+void integrate_kn_loop(const Dims &d, const KnArgs &args, const T *M, T *x_out, i64 *iter_out,
+                       double *err_out) {
+  constexpr i64 kLoopChunk = 512;
+  const i64 l = d.l, Nl = d.Nl, ll = l * l, sz = Nl * 4 * l;
+  const T ninv = T(1) / T(d.N);
+  const int mode = kn_mode();
+  DBuf<T> sbuf(2 * sz);
+  KnLoop<T> loop(l, Nl);
+  double *slot = static_cast<double *>(pinned_slot(0));
+  i64 done = 0;
+  bool resume = false;
+  int cur = 0;
+  double h[4];
+  for (;;) {
+    T *S = sbuf.get() + cur * sz;
+    loop.run(M, ninv, S, resume, done, args.maxit, trace_on() ? 1 : kLoopChunk, args.tol, mode,
+             slot);
+    pinned_slot_record(0);
+    read_back_wait(0, h, sizeof(h));
+    ISVD_CHECK(h[3] != 2.0, "KN: a grid barrier of the loop timed out");
+    if (trace_on() && (i64)h[1] > done)
+      std::fprintf(stderr, "isvd KN iter %lld err %.17g rho %.3g (loop)\n", (i64)h[1], h[0], h[2]);
+    done = (i64)h[1];
+    if (h[3] == 0.0) break;
+    resume = true;
+    if (h[3] == 1.0) {
+      // one iteration from this state, whose G is valid, by the eigendecomposition
+      const i64 want = Nl / 64 > 0 ? (Nl / 64 < 64 ? Nl / 64 : 64) : 1;
+      DBuf<T> ddg(2 * ll), w3(6 * ll), scal(4), parts((want + 1) * 2 * ll),
+          cwork(kn_chain_work_size(l));
+      DBuf<unsigned long long> bar(kKnChainBarWords);
+      KnChainWork<T> chain;
+      chain.buf = cwork.get();
+      chain.bar = bar.get();
+      kn_chain_init<T>(chain, (int)l);
+      const T *B = S + Nl * l;
+      const int nparts =
+          gemm_partials<T>('T', 'N', l, 2 * l, Nl, B, Nl, B, Nl, parts.get(), (int)want);
+      kn_eig_w3<T>(l, ninv, parts.get(), nparts, ddg.get(), chain, w3.get(), scal.get());
+      cur ^= 1;
+      gemm_shortk<T>('N', 'N', Nl, l, 2 * l, T(1), S, Nl, w3.get(), 2 * l, T(0),
+                     sbuf.get() + cur * sz, Nl, 3, Nl * l, 2 * ll, Nl * l);
+      h[0] = (double)read_scalar(scal.get());
+      ++done;
+      if (trace_on())
+        std::fprintf(stderr, "isvd KN iter %lld err %.17g (eig)\n", done, h[0]);
+      if (h[0] <= args.tol || done == args.maxit) break;
+    }
+  }
+  omatcopy<T>('N', Nl, l, T(1), sbuf.get() + cur * sz, Nl, x_out, Nl);
+  *iter_out = h[0] <= args.tol ? done : done + 1;
+  *err_out = h[0];
+}
+
 // The KN iteration in sketch coordinates.  A state [X | B | Bg | G] (Nl x 4l) holds X_c,
 // B_c = Qs^T Q_c, Bg_c = M B_c / N and G_c = M Bg_c / N; [D | Dg] = B_c^T [B_c | Bg_c] / N.
 // Iteration it, from state s to state s+1 (three states in a ring):
@@ -372,6 +463,10 @@ void integrate_kn_coords(const Dims &d, const KnArgs &args, const T *M, T *x_out
   const i64 l = d.l, Nl = d.Nl, ll = l * l;
   ISVD_CHECK(!ms || (std::is_same_v<T, float> && ms->n == Nl),
              "KN: the BF16-split M is for the FP32 loop with n = Nl");
+  if (!ms && kn_loop_takes<T>(l, Nl)) {
+    integrate_kn_loop<T>(d, args, M, x_out, iter_out, err_out);
+    return;
+  }
   // out := alpha M in (Nl x l, ld Nl)
   auto m_apply = [&](const T *in, T alpha, T *out) {
     if constexpr (std::is_same_v<T, float>) {
@@ -398,8 +493,6 @@ void integrate_kn_coords(const Dims &d, const KnArgs &args, const T *M, T *x_out
   chain.buf = cwork.get();
   chain.bar = bar.get();
   kn_chain_init<T>(chain, (int)l);
-  // eigendecomposition path
-  DBuf<T> w(l), zv(ll), zs(ll), zi(ll), c(ll), cinv(ll);
   const JoinAux join_aux;  // destroyed before the buffers above
   auto X = [&](i64 q) { return sbuf.get() + (q % 3) * sz; };
   auto B = [&](i64 q) { return X(q) + Nl * l; };
@@ -475,21 +568,7 @@ void integrate_kn_coords(const Dims &d, const KnArgs &args, const T *M, T *x_out
       HIP_CHECK(hipStreamSynchronize(ctx().aux));
       const i64 q = it - 1;
       gram(q);
-      kn_chain<T>((int)l, ninv, parts.get(), nparts, ddg.get(), chain, w3.get(), scal.get(), 1);
-      syev_small<T>(l, chain.Z(), l, w.get(), zv.get(), l);
-      hipLaunchKernelGGL(kn_scalars_kernel<T>, dim3(1), dim3(256), 0, ctx().stream, (int)l,
-                         (const T *)w.get(), (const T *)zv.get(), zs.get(), zi.get(), scal.get());
-      LAUNCH_CHECK();
-      small_gemm<T>('N', 'T', l, l, l, T(1), zs.get(), l, zs.get(), l, T(0), c.get(), l);
-      small_gemm<T>('N', 'T', l, l, l, T(1), zi.get(), l, zi.get(), l, T(0), cinv.get(), l);
-      hipLaunchKernelGGL(sym_from_upper_kernel<T>, dim3(grid_for(ll)), dim3(256), 0,
-                         ctx().stream, (int)l, cinv.get(), l);
-      LAUNCH_CHECK();
-      // F [in C] := C - D inv(C)  (:218)
-      small_gemm<T>('N', 'N', l, l, l, T(-1), ddg.get(), l, cinv.get(), l, T(1), c.get(), l);
-      hipLaunchKernelGGL(kn_assemble_kernel<T>, dim3(grid_for(ll)), dim3(256), 0, ctx().stream,
-                         (int)l, (const T *)c.get(), (const T *)cinv.get(), ninv, w3.get());
-      LAUNCH_CHECK();
+      kn_eig_w3<T>(l, ninv, parts.get(), nparts, ddg.get(), chain, w3.get(), scal.get());
       HIP_CHECK(hipEventRecord(ctx().join, ctx().stream));  // G_c is already in the state
       updates(q);
       read_back(h, scal.get(), sizeof(T));

@@ -82,6 +82,9 @@ void stage_post_symmetric(const Dims &d, char ordera, const T *a, i64 lda, const
 // its two BF16 terms instead (ms != nullptr, M unused): it then iterates with M'' = Mh + Ml and
 // forms its products with M on the BF16 matrix cores (split_sym_apply).
 struct SplitSym;
+// Whether integrate_kn_coords runs the loop on M itself in one launch (ms is then not needed).
+template <typename T>
+bool kn_loop_takes(i64 l, i64 Nl);
 template <typename T>
 void integrate_kn_coords(const Dims &d, const KnArgs &args, const T *M, T *x_out, i64 *iter,
                          double *err, const SplitSym *ms = nullptr);
