@@ -692,6 +692,12 @@ inline bool dl_eligible(const GemmArgs<double> &g, bool KA, bool KB, i64 batch) 
   return true;
 }
 
+}  // namespace isvd
+
+#include "gemm_thin.hpp"
+
+namespace isvd {
+
 // C = alpha * sum_s W[s] + beta * C  (fixed summation order -> deterministic).
 template <typename T>
 __global__ void splitk_reduce_kernel(i64 m, i64 n, int ksplit, const T *__restrict__ W,
@@ -736,6 +742,17 @@ __global__ void scale_kernel(i64 m, i64 n, T beta, T *C, i64 ldc, i64 sC) {
 namespace {
 
 constexpr int kTargetBlocks = 1024;  // ~4 workgroups per CU on 256 CUs
+
+// Sum of the K chunks' partials in g.W into C.
+template <typename T>
+void splitk_reduce(const GemmArgs<T> &g, i64 batch) {
+  int blocks = (int)((g.m * g.n + 255) / 256);
+  if (blocks > 4096) blocks = 4096;
+  hipLaunchKernelGGL(splitk_reduce_kernel<T>, dim3(blocks, (unsigned)batch), dim3(256), 0,
+                     ctx().stream, g.m, g.n, g.ksplit, (const T *)g.W, g.alpha, g.beta, g.C, g.ldc,
+                     g.sC, g.ct);
+  LAUNCH_CHECK();
+}
 
 template <typename T, bool TA, bool TB, int BM, int BN, int BK, int WGM, int WGN>
 void launch_cfg(GemmArgs<T> g, i64 batch) {
@@ -822,15 +839,7 @@ void launch_cfg(GemmArgs<T> g, i64 batch) {
     hipLaunchKernelGGL((gemm_kernel<T, TA, TB, BM, BN, BK, WGM, WGN>), grid,
                        dim3(64 * WGM * WGN), 0, ctx().stream, g);
   LAUNCH_CHECK();
-  if (ksplit > 1) {
-    const i64 mn = g.m * g.n;
-    int blocks = (int)((mn + 255) / 256);
-    if (blocks > 4096) blocks = 4096;
-    hipLaunchKernelGGL(splitk_reduce_kernel<T>, dim3(blocks, (unsigned)batch), dim3(256), 0,
-                       ctx().stream, g.m, g.n, ksplit, (const T *)g.W, g.alpha, g.beta, g.C,
-                       g.ldc, g.sC, g.ct);
-    LAUNCH_CHECK();
-  }
+  if (ksplit > 1) splitk_reduce(g, batch);
 }
 
 // 64 x 64 tiles with a given number of K chunks and no other choice made: the caller either
@@ -866,8 +875,55 @@ int fixed64(char transa, char transb, GemmArgs<T> g, i64 batch, int ksplit) {
   return launch_fixed64<T, true, true>(g, batch, ksplit);
 }
 
+// Few rows against a large op(B): gemm_thin_kernel, from K = 1024 and n = 256 on (below, a product
+// is a few microseconds either way).  FP32 with more than 48 rows only from 2^26 elements of B on:
+// a 3001 x 8191 B with unaligned columns takes 73 us against 69 us on 64 x 64 tiles there (59 / 68
+// at 48 rows; FP64 83 / 106 at 64).
+template <typename T>
+bool thin_eligible(const GemmArgs<T> &g, i64 batch) {
+  if (g.ct || g.upper || g.m > 64 || g.n < 256 || g.k < 1024 || batch > 1024) return false;
+  return sizeof(T) == 8 || g.m <= 48 || g.n * g.k >= (1ll << 26);
+}
+
+template <typename T, bool KB>
+void launch_thin(GemmArgs<T> g, i64 batch) {
+  using X = thin::Traits<T>;
+  const i64 blocks = (g.n + X::COLS - 1) / X::COLS;
+  // one workgroup per CU; a chunk of at least 8 groups of steps, and partial sums (written and
+  // read) below half of B's bytes
+  i64 ks = (256 + blocks * batch - 1) / (blocks * batch);
+  const i64 by_k = g.k / (8 * X::U * X::STEP), by_bytes = g.k / (4 * g.m);
+  if (ks > by_k) ks = by_k;
+  if (ks > by_bytes) ks = by_bytes;
+  if (ctx().max_wgs > 0)
+    while (ks > 1 && blocks * batch * ks > ctx().max_wgs) --ks;
+  const size_t per = sizeof(T) * (size_t)(batch * g.m * g.n);
+  while (ks > 1 && per * (size_t)ks > splitk_budget()) --ks;
+  if (ks < 1) ks = 1;
+  i64 kchunk = (g.k + ks - 1) / ks;
+  kchunk = (kchunk + X::STEP - 1) / X::STEP * X::STEP;
+  ks = (g.k + kchunk - 1) / kchunk;
+  g.ksplit = (int)ks;
+  g.kchunk = kchunk;
+  if (ks > 1) g.W = static_cast<T *>(splitk_workspace(per * (size_t)ks));
+  const dim3 grid((unsigned)blocks, (unsigned)(batch * ks));
+  const int mt = (int)((g.m + 15) / 16);
+  if (mt == 1) hipLaunchKernelGGL((gemm_thin_kernel<T, KB, 1>), grid, dim3(thin::NT), 0, ctx().stream, g);
+  else if (mt == 2) hipLaunchKernelGGL((gemm_thin_kernel<T, KB, 2>), grid, dim3(thin::NT), 0, ctx().stream, g);
+  else if (mt == 3) hipLaunchKernelGGL((gemm_thin_kernel<T, KB, 3>), grid, dim3(thin::NT), 0, ctx().stream, g);
+  else hipLaunchKernelGGL((gemm_thin_kernel<T, KB, 4>), grid, dim3(thin::NT), 0, ctx().stream, g);
+  LAUNCH_CHECK();
+  if (ks > 1) splitk_reduce(g, batch);
+}
+
 template <typename T, bool TA, bool TB>
 void launch(GemmArgs<T> g, i64 batch) {
+  if constexpr (!TA) {
+    if (thin_eligible(g, batch)) {
+      launch_thin<T, !TB>(g, batch);
+      return;
+    }
+  }
   const bool big = (g.m >= 128 && g.n >= 128);
   if (!big) {
     launch_cfg<T, TA, TB, 64, 64, 16, 2, 2>(g, batch);
