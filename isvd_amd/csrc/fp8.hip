@@ -55,42 +55,81 @@ __device__ inline float block_scale(float amax) {
   return ldexpf(1.f, e);
 }
 
-__global__ __launch_bounds__(256) void quantize_kernel(char ordera, i64 m, i64 n,
-                                                       const float *__restrict__ a, i64 lda,
-                                                       uint8_t *__restrict__ a8, i64 lda8,
+// One workgroup per 128 x 128 block, held in registers between the maximum and the encoding (64
+// values a thread, 16 loads of 16 bytes in flight), so that A is read once and nothing but the
+// codes of a column-major A passes through LDS.  Bound by reading 4 and writing 1 byte per
+// element: 131072 x 16384 FP32 in 1.98 ms, 5.4 TB/s, column-major 2.11 ms (10.5 ms through an FP32 tile in LDS with 4-byte loads and a
+// workgroup barrier between its column-strided writes and reads).
+//   row-major: 32 threads by 4 columns cover a row of the block, 8 rows a pass; a thread's 4 codes
+//   are one dword of the row.
+//   column-major: 32 threads by 4 rows cover a column; a thread holds 4 x 4 patches, whose 4 rows of
+//   4 codes go to LDS as dwords and leave as 16-byte row pieces.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+template <bool COLMAJOR>
+__global__ __launch_bounds__(256) void quantize_kernel(i64 m, i64 n, const float *__restrict__ a,
+                                                       i64 lda, uint8_t *__restrict__ a8, i64 lda8,
                                                        float *__restrict__ scale, i64 lds) {
-  __shared__ float tile[128][129];
+  constexpr int PITCH = 36;  // dwords per row of codes in LDS (rows stay 16-byte aligned)
+  __shared__ __align__(16) unsigned codes[COLMAJOR ? 128 * PITCH : 1];
   __shared__ float wmax[4];
   const i64 i0 = (i64)blockIdx.y * 128, j0 = (i64)blockIdx.x * 128;
-  const int t = threadIdx.x;
+  const int t = threadIdx.x, f = t & 31, q = t >> 5;
+  const bool whole = i0 + 128 <= m && j0 + 128 <= n;
+  // v[p][c]: row-major, row 8 p + q, column 4 f + c;
+  // column-major, p = 4 u + w: row 4 f + c, column 32 u + 4 q + w
+  f32x4 v[16];
   float amax = 0.f;
-  for (int e = t; e < 128 * 128; e += 256) {
-    const int fast = e & 127, slow = e >> 7;
-    const int ii = ordera == 'R' ? slow : fast, jj = ordera == 'R' ? fast : slow;
-    const i64 gi = i0 + ii, gj = j0 + jj;
-    float v = 0.f;
-    if (gi < m && gj < n) v = ordera == 'R' ? a[gi * lda + gj] : a[gi + gj * lda];
-    tile[ii][jj] = v;
-    amax = fmaxf(amax, fabsf(v));
+#pragma unroll
+  for (int p = 0; p < 16; ++p) {
+    const i64 fast = (COLMAJOR ? i0 : j0) + 4 * f;
+    const i64 slow = COLMAJOR ? j0 + 32 * (p >> 2) + 4 * q + (p & 3) : i0 + 8 * p + q;
+    const float *src = a + slow * lda + fast;
+    if (whole) {
+      v[p] = *reinterpret_cast<const f32x4u *>(src);
+    } else {
+      const i64 nf = COLMAJOR ? m : n, ns = COLMAJOR ? n : m;
+      for (int c = 0; c < 4; ++c) v[p][c] = (slow < ns && fast + c < nf) ? src[c] : 0.f;
+    }
   }
+#pragma unroll
+  for (int p = 0; p < 16; ++p)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) amax = fmaxf(amax, fabsf(v[p][c]));
   for (int o = 32; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o));
   if ((t & 63) == 0) wmax[t >> 6] = amax;
   __syncthreads();
   amax = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
   const float s = block_scale(amax), inv = 1.f / s;
   if (t == 0) scale[(i64)blockIdx.y * lds + blockIdx.x] = s;
-  // 128 rows x 8 chunks of 16 codes; columns >= n hold zeros (code 0)
-  for (int q = t; q < 128 * 8; q += 256) {
-    const int ii = q >> 3, c = q & 7;
-    const i64 gi = i0 + ii, gj = j0 + 16 * c;
-    if (gi >= m || gj >= n) continue;
-    u32x4 w;
-    for (int word = 0; word < 4; ++word) {
-      unsigned v = 0;
-      for (int b = 0; b < 4; ++b) v |= e4m3_code(tile[ii][16 * c + 4 * word + b] * inv) << (8 * b);
-      w[word] = v;
+  // rows are written to column roundup(n, 16); columns >= n hold zeros (code 0)
+  const i64 n16 = (n + 15) / 16 * 16;
+  if constexpr (!COLMAJOR) {
+#pragma unroll
+    for (int p = 0; p < 16; ++p) {
+      unsigned w = 0;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) w |= e4m3_code(v[p][c] * inv) << (8 * c);
+      const i64 gi = i0 + 8 * p + q, gj = j0 + 4 * f;
+      if (gi < m && gj < n16) *reinterpret_cast<unsigned *>(a8 + gi * lda8 + gj) = w;
     }
-    *reinterpret_cast<u32x4 *>(a8 + gi * lda8 + gj) = w;
+  } else {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        unsigned w = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w |= e4m3_code(v[4 * u + j][c] * inv) << (8 * j);
+        codes[(4 * f + c) * PITCH + 8 * u + q] = w;
+      }
+    __syncthreads();
+    for (int e = t; e < 128 * 8; e += 256) {
+      const int ii = e >> 3, c = e & 7;
+      const i64 gi = i0 + ii, gj = j0 + 16 * c;
+      if (gi < m && gj < n)
+        *reinterpret_cast<u32x4 *>(a8 + gi * lda8 + gj) =
+            *reinterpret_cast<const u32x4 *>(codes + ii * PITCH + 4 * c);
+    }
   }
 }
 
@@ -392,8 +431,13 @@ void quantize_e4m3(char ordera, i64 m, i64 n, const float *a, i64 lda, uint8_t *
   const i64 nbi = (m + 127) / 128, nbj = (n + 127) / 128;
   ISVD_CHECK(lds >= nbj, "ldscale (%lld) must be >= ceil(n / 128) (%lld)", lds, nbj);
   ISVD_CHECK(nbi <= 65535 && nbj <= 0x7FFFFFFF, "matrix too large for the quantizer grid");
-  hipLaunchKernelGGL(quantize_kernel, dim3((unsigned)nbj, (unsigned)nbi), dim3(256), 0,
-                     ctx().stream, ordera, m, n, a, lda, a8, lda8, scale, lds);
+  const dim3 grid((unsigned)nbj, (unsigned)nbi);
+  if (ordera == 'C')
+    hipLaunchKernelGGL(quantize_kernel<true>, grid, dim3(256), 0, ctx().stream, m, n, a, lda, a8,
+                       lda8, scale, lds);
+  else
+    hipLaunchKernelGGL(quantize_kernel<false>, grid, dim3(256), 0, ctx().stream, m, n, a, lda, a8,
+                       lda8, scale, lds);
   LAUNCH_CHECK();
 }
 
