@@ -25,9 +25,11 @@ __device__ __forceinline__ float dpp_mov(float v) {
 // Sum over the 16 lanes of a row, every lane receiving the same (bitwise) total: pairs
 // (quad_perm 1,0,3,2), quads (quad_perm 2,3,0,1), half rows (row_half_mirror), rows
 // (row_mirror).  Each step adds two partial sums in both orders, which FP addition makes equal.
-// All 16 lanes of the row must be active.
+// All 16 lanes of the row must be active.  (Contraction is off: with v a product, its addition
+// would become a fused one that rounds v of one lane only, and the lanes' totals would differ.)
 template <typename T>
 __device__ __forceinline__ T row16_sum(T v) {
+#pragma clang fp contract(off)
   v += dpp_mov<0xB1>(v);
   v += dpp_mov<0x4E>(v);
   v += dpp_mov<0x141>(v);
@@ -39,6 +41,7 @@ __device__ __forceinline__ T row16_sum(T v) {
 // every lane receiving the total.
 template <typename T>
 __device__ __forceinline__ T lane_group_sum(T v, int width) {
+#pragma clang fp contract(off)
   if (width >= 2) v += dpp_mov<0xB1>(v);
   if (width >= 4) v += dpp_mov<0x4E>(v);
   if (width >= 8) v += dpp_mov<0x141>(v);

@@ -2,12 +2,22 @@
 // the Gramian eigendecompositions of orthogonalization / postprocessing (gesvd of a PSD
 // matrix), the SVD of the TSQR R factor, and the KN eigendecomposition of Z.
 //
-// Method: one-sided (Hestenes) Jacobi with the round-robin parallel ordering.  One workgroup
-// owns one matrix, held column-major in LDS (128 x 128 FP64 = 128 KiB of the 160 KiB LDS).
-// Each round pairs all columns (n/2 disjoint pairs); a group of lanes per pair computes the
-// three dot products with a shuffle reduction, forms the rotation that orthogonalizes the two
-// columns, and applies it (and, optionally, to the right factor V kept in global memory).
-// A sweep with no rotation above the relative threshold ends the iteration.
+// Method: one-sided (Hestenes) Jacobi, parallel round-robin ordering over blocks of two columns.
+// One workgroup owns one matrix, held column-major in LDS (128 x 128 FP64 = 128 KiB of the 160
+// KiB LDS).  A group of 16 lanes holds the four columns of a block pair in registers through the
+// two rounds of cross rotations (and, at the start of a sweep, the one inside the blocks), two
+// rotations side by side in each, so that LDS traffic, the workgroup barrier and the wait for both
+// are paid every second round.  A sweep with no rotation above the relative threshold ends the
+// iteration.  The right factor is not accumulated on the way: the rotations go to a log and
+// are replayed on the rows of V by a second kernel, every row in registers of its own lanes.
+// A PSD matrix is factored by Cholesky in place first, W = L L^T, and the iteration runs on L,
+// whose singular values are the roots of W's: 9-10 sweeps instead of 13-15.
+//
+// Measured, FP64 (one rotation a round with the vectors of V in global memory before): V and U at
+// l = 64 660 -> 346 + 47 us, l = 128 3570 -> 1570 + 106 us; PSD at l = 48 450 -> 190 us, l = 128
+// 3000 -> 1250 us.  Bound by instruction issue: the vector unit is busy 50 % (l = 64, one wave per
+// SIMD) to 60 % (l = 128, two) of the time, the rest waits for LDS, barriers and dependent FP64
+// results; four groups of lanes per pair instead of two, or eight lanes a group, were slower.
 #include "la.hpp"
 
 #include <type_traits>
@@ -25,19 +35,24 @@ template <> struct Eps<double> { static constexpr double v = DBL_EPSILON; };
 template <> struct Eps<float> { static constexpr float v = FLT_EPSILON; };
 
 constexpr int kMaxSweeps = 40;
-// 16 lanes per column pair, each holding every 16th row of the pair's two columns: 4 pairs per
-// wave and, at n = 128, 16 waves (4 per SIMD), which hide each other's LDS, DPP, division and
-// (with V) global-memory latencies.  A round is bound by instruction issue and latency together:
-// 8 lanes per pair (8 waves) and 4 lanes (4 waves) were measured slower at n = 128.
+// 16 lanes per block pair, each holding every 16th row of its four columns
 constexpr int kTpp = 16;
-constexpr int kMaxThreads = 1024;
+constexpr int kMaxThreads = 512;  // n = 128: 32 groups
 
-// rows per lane for an n x n problem with tpp lanes per pair (a power of two, n <= tpp rows)
-inline int jacobi_rpl(i64 n, int tpp) {
+// the hardware's approximations (FP64: about 1e-8 relative; FP32: 1 ulp)
+__device__ __forceinline__ double rcp_approx(double x) { return __builtin_amdgcn_rcp(x); }
+__device__ __forceinline__ double rsq_approx(double x) { return __builtin_amdgcn_rsq(x); }
+__device__ __forceinline__ float rcp_approx(float x) { return __builtin_amdgcn_rcpf(x); }
+__device__ __forceinline__ float rsq_approx(float x) { return __builtin_amdgcn_rsqf(x); }
+
+// rows per lane for an n x n problem (a power of two)
+inline int jacobi_rpl(i64 n) {
   int r = 1;
-  while (r * tpp < n) r *= 2;
+  while (r * kTpp < n) r *= 2;
   return r;
 }
+// groups (block pairs) of an n-column problem: blocks of two columns, an even number of them
+__host__ __device__ inline int jacobi_groups(int n) { return (n + 3) / 4; }
 
 // round-robin (circle method) pairing of np players (np even), round r in [0, np-1), table
 // k in [0, np/2): player m = np - 1 stays at table 0, the others turn (r, k < m: no modulo)
@@ -52,22 +67,37 @@ __device__ __forceinline__ void rr_pair(int np, int r, int k, int &p, int &q) {
   }
 }
 
-// mode 0: SVD of A (general n x n).  mode 1: symmetric eigendecomposition of the matrix whose
+// The rotation log of one problem, 2 g slots a sweep (g groups) of four times g rotations: in slot
+// 0, for group k, the two rotations inside the blocks it starts with, (p0, p1), (q0, q1); in slot
+// 1 + r, r < 2 g - 1, the four cross rotations of its block pair in outer round r, (p0, q0),
+// (p1, q1), (p0, q1), (p1, q0).
+template <typename T>
+struct Rot {
+  T c, s;
+};
+__host__ __device__ inline i64 log_entries(int groups) {
+  return (i64)kMaxSweeps * 2 * groups * groups * 4;
+}
+
+enum { kGeneral = 0, kSymmetric = 1, kPsd = 2 };
+
+// kGeneral: SVD of A (general n x n).  kSymmetric: symmetric eigendecomposition of the matrix whose
 // upper triangle is stored in A, computed as the SVD of sym(A) + c I with c = 2 ||sym(A)||_F.
-// TPP lanes per pair, RPL rows per lane; the columns are padded with zero rows to TPP RPL
-// (rotations keep them zero), so the round loop has no row bounds.  Vwork holds V with the same
-// padded rows (TPP RPL x n).  blockDim.x = TPP lanes per pair, rounded up to whole waves.
-template <typename T, bool WANT_V, int TPP, int RPL>
+// kPsd: SVD of a symmetric positive semi-definite A (upper triangle), by the SVD of its Cholesky
+// factor where every pivot stays above rounding, else of A itself.
+// The columns are padded with zero rows to 16 RPL and with zero columns to 4 groups (rotations
+// keep both zero), so the round loop has no bounds.  blockDim.x = 16 lanes per group, rounded up
+// to whole waves.
+template <typename T, int RPL>
 __global__ __launch_bounds__(kMaxThreads) void svd_jacobi_kernel(
     int n, int mode, const T *__restrict__ A, i64 lda, i64 sA, T *__restrict__ sig, i64 lds,
-    T *__restrict__ U, i64 ldu, i64 sU, T *__restrict__ Vwork, T *__restrict__ V, i64 ldv,
-    i64 sV, T *__restrict__ shift_out) {
+    T *__restrict__ U, i64 ldu, i64 sU, Rot<T> *__restrict__ log, int *__restrict__ order,
+    T *__restrict__ shift_out) {
   extern __shared__ unsigned char smem_raw[];
-  // n x n, leading dimension n + 1: the columns of the pairs a wave works on start in
-  // different banks
+  // leading dimension 16 RPL + 1: the columns a wave works on start in different banks
   T *G = reinterpret_cast<T *>(smem_raw);
   __shared__ T red[kMaxThreads / 64];
-  __shared__ T nrm[128];
+  __shared__ T nrm[128];  // squared column norms during the sweeps, then the norms
   __shared__ int rank_of[128];
   __shared__ int n_rot;
   __shared__ T shift_sh;
@@ -76,27 +106,25 @@ __global__ __launch_bounds__(kMaxThreads) void svd_jacobi_kernel(
   const int tid = threadIdx.x;
   const int nt = blockDim.x, waves = nt / 64;
   const T *Ab = A + (i64)b * sA;
-  const int np = (n + 1) & ~1;
-  const int npairs = np / 2;
-  const int grp = tid / TPP, sub = tid % TPP;
-  constexpr int R = TPP * RPL;  // padded rows
+  const int groups = jacobi_groups(n), cols = 4 * groups, blocks = 2 * groups;
+  const int grp = tid / kTpp, sub = tid % kTpp;
+  const bool live = grp < groups;
+  constexpr int R = kTpp * RPL;  // padded rows
   constexpr int ld = R + 1;
 
-  // ---- load (rows n .. R-1 zero) ----
-  for (int e = tid; e < R * n; e += nt) {
-    const int i = e % R, j = e / R;
-    T v = T(0);
-    if (i < n) {
-      if (mode == 1) {
-        v = (i <= j) ? Ab[i + (i64)j * lda] : Ab[j + (i64)i * lda];  // symmetric from upper
-      } else {
-        v = Ab[i + (i64)j * lda];
-      }
+  // ---- load (rows n .. R-1 and columns n .. zero) ----
+  auto load = [&](bool upper) {
+    for (int e = tid; e < R * cols; e += nt) {
+      const int i = e % R, j = e / R;
+      T v = T(0);
+      if (i < n && j < n)
+        v = (upper && i > j) ? Ab[j + (i64)i * lda] : Ab[i + (i64)j * lda];
+      G[i + j * ld] = v;
     }
-    G[i + j * ld] = v;
-  }
-  __syncthreads();
-  if (mode == 1) {
+    __syncthreads();
+  };
+  load(mode != kGeneral);
+  if (mode == kSymmetric) {
     // c = 2 ||A||_F (+1 when A == 0), deterministic block reduction
     T part = 0;
     for (int e = tid; e < n * n; e += nt) {
@@ -117,84 +145,162 @@ __global__ __launch_bounds__(kMaxThreads) void svd_jacobi_kernel(
     for (int i = tid; i < n; i += nt) G[i + i * ld] += shift_sh;
     __syncthreads();
   }
-  T *Vb = WANT_V ? (Vwork + (i64)b * R * n) : nullptr;
-  if (WANT_V) {
-    for (int e = tid; e < R * n; e += nt) {
-      const int i = e % R, j = e / R;
-      Vb[e] = (i == j) ? T(1) : T(0);
-    }
+  bool factored = false;
+  if (mode == kPsd) {
+    // L D L^T in place, right-looking on the lower triangle, one barrier a step (column k stays
+    // unscaled until the end); a pivot not above n u A(k, k) is rounding, and A is taken itself
+    for (int j = tid; j < n; j += nt) nrm[j] = Eps<T>::v * T(n) * G[j + j * ld];
     __syncthreads();
-  }
-
-  const T tol = Eps<T>::v * T(n);
-  for (int sweep = 0; sweep < kMaxSweeps; ++sweep) {
-    if (tid == 0) n_rot = 0;
-    __syncthreads();
-    for (int r = 0; r < np - 1; ++r) {
-      int p = n, q = n;
-      if (grp < npairs) rr_pair(np, r, grp, p, q);
-      if (p < n && q < n) {
-        // the V columns are requested first: their latency runs under the dot products
-        T vp[RPL], vq[RPL];
-        const T *vcp = Vb + (i64)p * R + sub, *vcq = Vb + (i64)q * R + sub;
-        if (WANT_V) {
-#pragma unroll
-          for (int u = 0; u < RPL; ++u) {
-            vp[u] = vcp[u * TPP];
-            vq[u] = vcq[u * TPP];
-          }
-        }
-        // the two columns stay in registers between the dot products and the rotation
-        T *cp = G + p * ld + sub, *cq = G + q * ld + sub;
-        T gp[RPL], gq[RPL];
-        T alpha = 0, beta = 0, gamma = 0;
-#pragma unroll
-        for (int u = 0; u < RPL; ++u) {
-          gp[u] = cp[u * TPP];
-          gq[u] = cq[u * TPP];
-          alpha += gp[u] * gp[u];
-          beta += gq[u] * gq[u];
-          gamma += gp[u] * gq[u];
-        }
-        alpha = lane_group_sum(alpha, TPP);
-        beta = lane_group_sum(beta, TPP);
-        gamma = lane_group_sum(gamma, TPP);
-        // |gamma| > tol sqrt(alpha beta), compared in squares
-        if (gamma != T(0) && gamma * gamma > tol * tol * (alpha * beta)) {
-          // t = sign(zeta) / (|zeta| + sqrt(1 + zeta^2)), zeta = (beta - alpha) / (2 gamma); in
-          // FP64 multiplied through by |2 gamma| (one division less on the round's dependent
-          // chain; the squares stay far from overflow at FP64 range), sign(zeta) = +1 at zeta = 0
-          T t;
-          if constexpr (std::is_same_v<T, double>) {
-            const T d = beta - alpha, g2 = T(2) * gamma;
-            const bool pos = d == T(0) || ((d > T(0)) == (g2 > T(0)));
-            t = (pos ? fabs(g2) : -fabs(g2)) / (fabs(d) + sqrt(d * d + g2 * g2));
-          } else {
-            const T zeta = (beta - alpha) / (T(2) * gamma);
-            t = (zeta >= T(0) ? T(1) : T(-1)) / (fabs(zeta) + sqrt(T(1) + zeta * zeta));
-          }
-          const T c = T(1) / sqrt(T(1) + t * t);
-          const T s = c * t;
-#pragma unroll
-          for (int u = 0; u < RPL; ++u) {
-            cp[u * TPP] = c * gp[u] - s * gq[u];
-            cq[u * TPP] = s * gp[u] + c * gq[u];
-          }
-          if (WANT_V) {
-            T *wp = Vb + (i64)p * R + sub, *wq = Vb + (i64)q * R + sub;
-#pragma unroll
-            for (int u = 0; u < RPL; ++u) {
-              wp[u * TPP] = c * vp[u] - s * vq[u];
-              wq[u * TPP] = s * vp[u] + c * vq[u];
-            }
-          }
-          if (sub == 0) atomicAdd(&n_rot, 1);
-        }
+    factored = true;
+    const int i = tid % R, jg = tid / R, js = nt / R;
+    for (int k = 0; k < n; ++k) {
+      const T d = G[k + k * ld];
+      if (!(d > nrm[k]) || !(d < T(INFINITY))) {
+        factored = false;
+        break;
+      }
+      const T w = T(1) / d;
+      if (jg < js && i > k && i < n) {
+        const T lik = G[i + k * ld] * w;
+        for (int j = k + 1 + jg; j <= i; j += js) G[i + j * ld] -= lik * G[j + k * ld];
       }
       __syncthreads();
     }
-    if (n_rot == 0) break;
+    if (factored) {
+      for (int e = tid; e < R * n; e += nt) {
+        const int r = e % R, j = e / R;
+        if (r != j) G[r + j * ld] = r > j ? G[r + j * ld] / sqrt(G[j + j * ld]) : T(0);
+      }
+      __syncthreads();
+      for (int j = tid; j < n; j += nt) G[j + j * ld] = sqrt(G[j + j * ld]);
+      __syncthreads();
+    } else {
+      __syncthreads();
+      load(true);
+    }
+  }
+
+  const T tol2 = (Eps<T>::v * T(n)) * (Eps<T>::v * T(n));
+  // Two rotations side by side, columns (a0, b0) and (a1, b1) with squared norms na, nb.  With
+  // zeta = (nb - na) / (2 gamma) = cot(2 theta): r = (1 + zeta^2)^(-1/2), c^2 = (1 + |zeta| r) / 2,
+  // s = sign(zeta) r / (2 c), from the reciprocal (square root) instructions as they are, to about
+  // 1e-8: an angle off by that leaves 1e-8 gamma behind, which the next sweep takes.  What has to
+  // be exact is c^2 + s^2 = 1: both are scaled by (1 + e)^(-1/2), e = c^2 + s^2 - 1, to third order.
+  // (Exact divisions and roots: 110 ns more a round.)
+  typedef T Col[RPL];
+  int rotated = 0;
+  auto rot2 = [&](Col &a0, Col &b0, T &na0, T &nb0, Col &a1, Col &b1, T &na1, T &nb1,
+                  Rot<T> *out) {
+    T g0 = 0, g1 = 0;
+#pragma unroll
+    for (int u = 0; u < RPL; ++u) {
+      g0 += a0[u] * b0[u];
+      g1 += a1[u] * b1[u];
+    }
+    g0 = lane_group_sum(g0, kTpp);
+    g1 = lane_group_sum(g1, kTpp);
+    // |gamma| > tol sqrt(alpha beta), compared in squares
+    const bool n0 = g0 * g0 > tol2 * (na0 * nb0), n1 = g1 * g1 > tol2 * (na1 * nb1);
+    Rot<T> r0{T(1), T(0)}, r1{T(1), T(0)};
+    if (n0 || n1) {
+      auto angle = [&](bool need, T g, T &na, T &nb) {
+        const T zeta = (nb - na) * rcp_approx(T(2) * g);
+        const T r = rsq_approx(T(1) + zeta * zeta);
+        const T c2 = T(0.5) + T(0.5) * fabs(zeta) * r;
+        const T y = rsq_approx(c2);
+        T c = c2 * y, s = T(0.5) * r * y;
+        const T e = c * c + (s * s - T(1));
+        const T f = T(1) + e * (T(0.375) * e - T(0.5));
+        c = need ? c * f : T(1);
+        s = need ? (zeta >= T(0) ? s * f : -(s * f)) : T(0);
+        const T g2 = T(2) * c * s * g, cc = c * c, ss = s * s;
+        const T xa = (cc * na - g2) + ss * nb, xb = (ss * na + g2) + cc * nb;
+        na = xa;
+        nb = xb;
+        return Rot<T>{c, s};
+      };
+      r0 = angle(n0, g0, na0, nb0);
+      r1 = angle(n1, g1, na1, nb1);
+#pragma unroll
+      for (int u = 0; u < RPL; ++u) {
+        const T x0 = a0[u], y0 = b0[u], x1 = a1[u], y1 = b1[u];
+        a0[u] = r0.c * x0 - r0.s * y0;
+        b0[u] = r0.s * x0 + r0.c * y0;
+        a1[u] = r1.c * x1 - r1.s * y1;
+        b1[u] = r1.s * x1 + r1.c * y1;
+      }
+      rotated = 1;
+    }
+    if (log && sub == 0 && live) {
+      out[0] = r0;
+      out[groups] = r1;
+    }
+  };
+  Rot<T> *lg = log ? log + (i64)b * log_entries(groups) : nullptr;
+  int sweep = 0;
+  for (; sweep < kMaxSweeps; ++sweep) {
+    if (tid == 0) n_rot = 0;
+    rotated = 0;
+    for (int r = 0; r < blocks - 1; ++r) {
+      int P = 0, Q = 1;
+      if (live) rr_pair(blocks, r, grp, P, Q);
+      Rot<T> *out = lg + ((i64)sweep * blocks + 1 + r) * 4 * groups + grp;
+      if (live) {
+        T *cp = G + 2 * P * ld + sub, *cq = G + 2 * Q * ld + sub;
+        Col p0, p1, q0, q1;
+#pragma unroll
+        for (int u = 0; u < RPL; ++u) {
+          p0[u] = cp[u * kTpp];
+          p1[u] = cp[ld + u * kTpp];
+          q0[u] = cq[u * kTpp];
+          q1[u] = cq[ld + u * kTpp];
+        }
+        T np0, np1, nq0, nq1;
+        if (r == 0) {
+          // squared norms afresh; within the sweep each rotation updates its two (a sweep without a
+          // rotation, which ends the iteration, thus tested every pair against norms of its
+          // columns); the rotations inside the blocks
+          np0 = np1 = nq0 = nq1 = T(0);
+#pragma unroll
+          for (int u = 0; u < RPL; ++u) {
+            np0 += p0[u] * p0[u];
+            np1 += p1[u] * p1[u];
+            nq0 += q0[u] * q0[u];
+            nq1 += q1[u] * q1[u];
+          }
+          np0 = lane_group_sum(np0, kTpp);
+          np1 = lane_group_sum(np1, kTpp);
+          nq0 = lane_group_sum(nq0, kTpp);
+          nq1 = lane_group_sum(nq1, kTpp);
+          rot2(p0, p1, np0, np1, q0, q1, nq0, nq1, lg + (i64)sweep * blocks * 4 * groups + grp);
+        } else {
+          np0 = nrm[2 * P];
+          np1 = nrm[2 * P + 1];
+          nq0 = nrm[2 * Q];
+          nq1 = nrm[2 * Q + 1];
+        }
+        rot2(p0, q0, np0, nq0, p1, q1, np1, nq1, out);
+        rot2(p0, q1, np0, nq1, p1, q0, np1, nq0, out + 2 * groups);
+#pragma unroll
+        for (int u = 0; u < RPL; ++u) {
+          cp[u * kTpp] = p0[u];
+          cp[ld + u * kTpp] = p1[u];
+          cq[u * kTpp] = q0[u];
+          cq[ld + u * kTpp] = q1[u];
+        }
+        // (every lane of the group writes the same four values)
+        nrm[2 * P] = np0;
+        nrm[2 * P + 1] = np1;
+        nrm[2 * Q] = nq0;
+        nrm[2 * Q + 1] = nq1;
+      }
+      __syncthreads();
+    }
+    if (rotated && sub == 0) n_rot = 1;
     __syncthreads();
+    const int go = n_rot;
+    __syncthreads();
+    if (go == 0) break;
   }
 
   // ---- singular values (column norms), ranks for descending order ----
@@ -215,8 +321,9 @@ __global__ __launch_bounds__(kMaxThreads) void svd_jacobi_kernel(
     rank_of[j] = rk;
   }
   __syncthreads();
-  for (int j = tid; j < n; j += nt) sig[(i64)b * lds + rank_of[j]] = nrm[j];
-  if (mode == 1 && tid == 0 && shift_out) shift_out[b] = shift_sh;
+  for (int j = tid; j < n; j += nt)
+    sig[(i64)b * lds + rank_of[j]] = factored ? nrm[j] * nrm[j] : nrm[j];
+  if (mode == kSymmetric && tid == 0 && shift_out) shift_out[b] = shift_sh;
   if (U) {
     T *Ub = U + (i64)b * sU;
     for (int e = tid; e < n * n; e += nt) {
@@ -225,14 +332,100 @@ __global__ __launch_bounds__(kMaxThreads) void svd_jacobi_kernel(
       Ub[i + (i64)rank_of[j] * ldu] = (sj > T(0)) ? G[i + j * ld] / sj : T(0);
     }
   }
-  if (WANT_V && V) {
-    __syncthreads();
-    T *Vo = V + (i64)b * sV;
-    for (int e = tid; e < n * n; e += nt) {
-      const int i = e % n, j = e / n;
-      Vo[i + (i64)rank_of[j] * ldv] = Vb[i + (i64)j * R];
+  if (order) {
+    // the columns' ranks, then the sweeps that rotated anything
+    for (int j = tid; j < n; j += nt) order[b * 132 + j] = rank_of[j];
+    if (tid == 0) order[b * 132 + 128] = sweep;
+  }
+}
+
+// V of the SVD from the rotation log: row i of V is e_i^T through the rotations in order.  A row
+// lives in the registers of `seg` lanes (a power of two >= groups), lane k holding the entries of
+// the block pair at table k, and between outer rounds the blocks move to the next table as the
+// players of the circle do: p to the left, q to the right, turning at both ends.  No barrier, no
+// LDS; the log is read eight outer rounds ahead.  128 x 128 FP64, 10 sweeps: 106 us (64 x 64: 47 us).
+template <typename T>
+__device__ __forceinline__ T from_next(T v) { return dpp_mov<0x130>(v); }  // lane i: lane i + 1's
+template <typename T>
+__device__ __forceinline__ T from_prev(T v) { return dpp_mov<0x138>(v); }  // lane i: lane i - 1's
+
+template <typename T>
+__global__ __launch_bounds__(256) void jacobi_replay_kernel(int n, int seg,
+                                                            const Rot<T> *__restrict__ log,
+                                                            const int *__restrict__ order,
+                                                            T *__restrict__ V, i64 ldv, i64 sV) {
+  const int groups = jacobi_groups(n), blocks = 2 * groups;
+  const int b = blockIdx.y, lane = threadIdx.x & 63;
+  const int k = lane % seg;  // table
+  const int row = (blockIdx.x * 4 + (threadIdx.x >> 6)) * (64 / seg) + lane / seg;
+  const int sweeps = order[b * 132 + 128];
+  const Rot<T> *lg = log + (i64)b * log_entries(groups);
+  const bool live = k < groups;
+  const int kc = live ? k : 0;
+  // the entries of this lane's blocks in round 0: P = k, Q = last block (k = 0) or blocks - 1 - k
+  const int P = kc, Q = kc == 0 ? blocks - 1 : blocks - 1 - kc;
+  T p0 = row == 2 * P, p1 = row == 2 * P + 1, q0 = row == 2 * Q, q1 = row == 2 * Q + 1;
+  auto rot = [](const Rot<T> &r, T &a, T &c) {
+    const T x = a, y = c;
+    a = r.c * x - r.s * y;
+    c = r.s * x + r.c * y;
+  };
+  constexpr int AHEAD = 8;
+  struct Slot {
+    Rot<T> r[4];
+  };
+  const int total = sweeps * blocks;
+  auto fetch = [&](int i) {
+    const int c = i < total ? i : total - 1;
+    Slot v;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v.r[j] = lg[((i64)c * 4 + j) * groups + kc];
+    return v;
+  };
+  if (total > 0) {
+    Slot buf[AHEAD];
+#pragma unroll
+    for (int a = 0; a < AHEAD; ++a) buf[a] = fetch(a);
+    int slot = 0;  // of the sweep
+    for (int i0 = 0; i0 < total; i0 += AHEAD) {
+#pragma unroll
+      for (int a = 0; a < AHEAD; ++a) {
+        const Slot s = buf[a];
+        buf[a] = fetch(i0 + a + AHEAD);
+        if (i0 + a < total) {
+          if (slot == 0) {
+            rot(s.r[0], p0, p1);
+            rot(s.r[1], q0, q1);
+          } else {
+            rot(s.r[0], p0, q0);
+            rot(s.r[1], p1, q1);
+            rot(s.r[2], p0, q1);
+            rot(s.r[3], p1, q0);
+            if (groups > 1) {
+              // p_k := p_{k+1}, p_last := q_last; q_k := q_{k-1} (k >= 2), q_1 := p_0; q_0 stays
+              const T np0 = from_next(p0), np1 = from_next(p1);
+              const T nq0 = from_prev(k == 0 ? p0 : q0), nq1 = from_prev(k == 0 ? p1 : q1);
+              const bool last = k == groups - 1;
+              const T lp0 = last ? q0 : np0, lp1 = last ? q1 : np1;
+              q0 = k == 0 ? q0 : nq0;
+              q1 = k == 0 ? q1 : nq1;
+              p0 = lp0;
+              p1 = lp1;
+            }
+          }
+          slot = slot + 1 == blocks ? 0 : slot + 1;
+        }
+      }
     }
   }
+  if (row >= n || !live) return;
+  // whole sweeps leave every block where it started
+  T *Vb = V + (i64)b * sV;
+  const int *rk = order + b * 132;
+  if (2 * P < n) Vb[row + (i64)rk[2 * P] * ldv] = p0;
+  if (2 * P + 1 < n) Vb[row + (i64)rk[2 * P + 1] * ldv] = p1;
+  if (2 * Q < n) Vb[row + (i64)rk[2 * Q] * ldv] = q0;
+  if (2 * Q + 1 < n) Vb[row + (i64)rk[2 * Q + 1] * ldv] = q1;
 }
 
 // eigenvalues ascending from the shifted SVD: w[j] = sig[n-1-j] - c, Z[:, j] = U[:, n-1-j]
@@ -247,50 +440,45 @@ __global__ void syev_finish_kernel(int n, const T *sig, const T *shift, const T 
   }
 }
 
-template <typename T, bool WANT_V, int TPP, int RPL>
-void launch_rpl(int nt, i64 n, int mode, const T *A, i64 lda, i64 sA, T *s, i64 lds, T *U,
-                i64 ldu, i64 sU, T *vwork, T *V, i64 ldv, i64 sV, i64 batch, T *shift_out) {
-  const size_t shmem = sizeof(T) * (size_t)(TPP * RPL + 1) * (size_t)n;
-  auto kern = svd_jacobi_kernel<T, WANT_V, TPP, RPL>;
+template <typename T, int RPL>
+void launch_rpl(i64 n, int mode, const T *A, i64 lda, i64 sA, T *s, i64 lds, T *U, i64 ldu, i64 sU,
+                i64 batch, Rot<T> *log, int *order, T *shift_out) {
+  const int groups = jacobi_groups((int)n);
+  const size_t shmem = sizeof(T) * (size_t)(kTpp * RPL + 1) * (size_t)(4 * groups);
+  const int nt = (groups * kTpp + 63) / 64 * 64;
+  auto kern = svd_jacobi_kernel<T, RPL>;
   HIP_CHECK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)shmem));
   hipLaunchKernelGGL(kern, dim3((unsigned)batch), dim3(nt), shmem, ctx().stream, (int)n, mode, A,
-                     lda, sA, s, lds, U, ldu, sU, vwork, V, ldv, sV, shift_out);
+                     lda, sA, s, lds, U, ldu, sU, log, order, shift_out);
   LAUNCH_CHECK();
-}
-
-template <typename T, bool WANT_V>
-void launch_v(i64 n, int mode, const T *A, i64 lda, i64 sA, T *s, i64 lds, T *U, i64 ldu, i64 sU,
-              T *vwork, T *V, i64 ldv, i64 sV, i64 batch, T *shift_out) {
-  constexpr int TPP = kTpp;
-  const i64 npairs = (n + 1) / 2;
-  const int nt = (int)((npairs * TPP + 63) / 64 * 64);
-#define ISVD_JAC(R) \
-  launch_rpl<T, WANT_V, TPP, R>(nt, n, mode, A, lda, sA, s, lds, U, ldu, sU, vwork, V, ldv, sV,   \
-                                batch, shift_out)
-  switch (jacobi_rpl(n, TPP)) {
-    case 1: ISVD_JAC(1); break;
-    case 2: ISVD_JAC(2); break;
-    case 4: ISVD_JAC(4); break;
-    case 8: ISVD_JAC(8); break;
-    default: ISVD_JAC(128 / TPP); break;
-  }
-#undef ISVD_JAC
 }
 
 template <typename T>
 void launch_svd(i64 n, int mode, const T *A, i64 lda, i64 sA, T *s, i64 lds, T *U, i64 ldu,
                 i64 sU, T *V, i64 ldv, i64 sV, i64 batch, T *shift_out) {
   ISVD_CHECK(n >= 1 && n <= 128, "small SVD supports 1 <= n <= 128 (got %lld)", n);
-  if (V) {
-    // V with its rows padded like the columns of the matrix (at most 128 rows)
-    DBuf<T> vwork(batch * (i64)kTpp * jacobi_rpl(n, kTpp) * n);
-    launch_v<T, true>(n, mode, A, lda, sA, s, lds, U, ldu, sU, vwork.get(), V, ldv, sV, batch,
-                      shift_out);
-  } else {
-    launch_v<T, false>(n, mode, A, lda, sA, s, lds, U, ldu, sU, (T *)nullptr, (T *)nullptr,
-                       (i64)0, (i64)0, batch, shift_out);
+  const int groups = jacobi_groups((int)n);
+  DBuf<Rot<T>> log(V ? batch * log_entries(groups) : 0);
+  DBuf<int> order(V ? batch * 132 : 0);
+#define ISVD_JAC(R)                                                                              \
+  launch_rpl<T, R>(n, mode, A, lda, sA, s, lds, U, ldu, sU, batch, log.get(), order.get(), shift_out)
+  switch (jacobi_rpl(n)) {
+    case 1: ISVD_JAC(1); break;
+    case 2: ISVD_JAC(2); break;
+    case 4: ISVD_JAC(4); break;
+    default: ISVD_JAC(8); break;
   }
+#undef ISVD_JAC
+  if (!V) return;
+  int seg = 1;
+  while (seg < groups) seg *= 2;
+  const int rows = 4 * (64 / seg);  // per workgroup
+  hipLaunchKernelGGL(jacobi_replay_kernel<T>,
+                     dim3((unsigned)((n + rows - 1) / rows), (unsigned)batch), dim3(256), 0,
+                     ctx().stream, (int)n, seg, (const Rot<T> *)log.get(),
+                     (const int *)order.get(), V, ldv, sV);
+  LAUNCH_CHECK();
 }
 
 }  // namespace
@@ -299,13 +487,20 @@ template <typename T>
 void svd_small(i64 n, T *A, i64 lda, i64 sA, T *s, i64 lds, T *U, i64 ldu, i64 sU, T *V,
                i64 ldv, i64 sV, i64 batch) {
   if (batch <= 0) return;
-  launch_svd<T>(n, 0, A, lda, sA, s, lds, U, ldu, sU, V, ldv, sV, batch, nullptr);
+  launch_svd<T>(n, kGeneral, A, lda, sA, s, lds, U, ldu, sU, V, ldv, sV, batch, nullptr);
+}
+
+template <typename T>
+void eig_psd_small(i64 n, const T *A, i64 lda, i64 sA, T *s, i64 lds, T *U, i64 ldu, i64 sU,
+                   i64 batch) {
+  if (batch <= 0) return;
+  launch_svd<T>(n, kPsd, A, lda, sA, s, lds, U, ldu, sU, (T *)nullptr, 0, 0, batch, nullptr);
 }
 
 template <typename T>
 void syev_small(i64 n, const T *A, i64 lda, T *w, T *Z, i64 ldz) {
   DBuf<T> sig(n), usrt(n * n), shift(1);
-  launch_svd<T>(n, 1, A, lda, 0, sig.get(), n, usrt.get(), n, 0, nullptr, 0, 0, 1, shift.get());
+  launch_svd<T>(n, kSymmetric, A, lda, 0, sig.get(), n, usrt.get(), n, 0, nullptr, 0, 0, 1, shift.get());
   hipLaunchKernelGGL(syev_finish_kernel<T>, dim3(ceil_div(n * n, 256)), dim3(256), 0,
                      ctx().stream, (int)n, (const T *)sig.get(), (const T *)shift.get(),
                      (const T *)usrt.get(), w, Z, ldz);
@@ -316,6 +511,9 @@ template void svd_small<double>(i64, double *, i64, i64, double *, i64, double *
                                 double *, i64, i64, i64);
 template void svd_small<float>(i64, float *, i64, i64, float *, i64, float *, i64, i64, float *,
                                i64, i64, i64);
+template void eig_psd_small<double>(i64, const double *, i64, i64, double *, i64, double *, i64, i64,
+                                    i64);
+template void eig_psd_small<float>(i64, const float *, i64, i64, float *, i64, float *, i64, i64, i64);
 template void syev_small<double>(i64, const double *, i64, double *, double *, i64);
 template void syev_small<float>(i64, const float *, i64, float *, float *, i64);
 

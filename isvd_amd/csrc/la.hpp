@@ -59,6 +59,13 @@ template <typename T>
 void svd_small(i64 n, T *A, i64 lda, i64 sA, T *s, i64 lds, T *U, i64 ldu, i64 sU, T *V,
                i64 ldv, i64 sV, i64 batch);
 
+// Eigendecomposition of symmetric positive semi-definite matrices (upper triangle read), as
+// svd_small's: eigenvalues descending in s, eigenvectors in U.  Runs on the Cholesky factor where
+// the matrix has one in working precision.
+template <typename T>
+void eig_psd_small(i64 n, const T *A, i64 lda, i64 sA, T *s, i64 lds, T *U, i64 ldu, i64 sU,
+                   i64 batch);
+
 // Symmetric eigendecomposition of n x n matrices (upper triangle referenced), LAPACK syev
 // conventions: eigenvalues ascending in w, eigenvectors in Z (n x n, ldz).  Built on
 // svd_small of the shifted matrix (A + c I, c >= |lambda|_max), which is positive

@@ -76,7 +76,7 @@ void stage_orth_gramian_b(const Dims &d, float *yst, i64 ldyst, bool cholqr) {
     gemm<float>('N', 'T', l, l, m, 1.f, src, lds, src, lds, 0.f, w32.get(), l, N, l, l, l * l);
     convert<double, float>(l, l * N, w32.get(), l, w64.get(), l);
     // W_i = U_i diag(s_i) U_i^T; U_i := U_i diag(s_i)^{-1/2}
-    svd_small<double>(l, w64.get(), l, l * l, s64.get(), l, u64.get(), l, l * l, nullptr, 0, 0, N);
+    eig_psd_small<double>(l, w64.get(), l, l * l, s64.get(), l, u64.get(), l, l * l, N);
     hipLaunchKernelGGL(colscale_rsqrt_kernel, dim3(grid_for(l * l), (unsigned)N), dim3(256), 0,
                        ctx().stream, (int)l, (const double *)s64.get(), u64.get());
     LAUNCH_CHECK();

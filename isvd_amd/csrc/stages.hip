@@ -277,7 +277,7 @@ void stage_orth_gramian(const Dims &d, T *yst, i64 ldyst, bool cholqr) {
   // W_i := Y_i^T Y_i  (:81-84)
   gemm<T>('N', 'T', l, l, m, T(1), yst, ldyst, yst, ldyst, T(0), w.get(), l, N, l, l, l * l);
   // gesvd('O','N') of every W_i  (:87-90)
-  svd_small<T>(l, w.get(), l, l * l, s.get(), l, u.get(), l, l * l, nullptr, 0, 0, N);
+  eig_psd_small<T>(l, w.get(), l, l * l, s.get(), l, u.get(), l, l * l, N);
   // s := sqrt(s); U_i := U_i / s_i  (:91, :94)
   hipLaunchKernelGGL(sqrt_and_colscale_kernel<T>, dim3(grid_for(l * l), (unsigned)N), dim3(256),
                      0, ctx().stream, (int)l, (int)l, (const T *)s.get(), l, u.get(), l, l * l);
@@ -794,7 +794,7 @@ void post_gramian_z(const Dims &d, const T *qt, i64 ldqt, T *zt, T *s, T *ut, i6
   DBuf<T> w(l * l), uw(l * l);
   // W := Z^T Z (:145); gesvd('O','N') + vSqrt (:149-151)
   gemm<T>('N', 'T', l, l, d.n, T(1), zt, l, zt, l, T(0), w.get(), l);
-  svd_small<T>(l, w.get(), l, 0, s, l, uw.get(), l, 0, nullptr, 0, 0, 1);
+  eig_psd_small<T>(l, w.get(), l, 0, s, l, uw.get(), l, 0, 1);
   hipLaunchKernelGGL(sqrt_inplace_kernel<T>, dim3(1, 1), dim3(256), 0, ctx().stream, (int)l, s);
   LAUNCH_CHECK();
   // U^T := W[:, :k]^T Qbar^T (:157-158)
