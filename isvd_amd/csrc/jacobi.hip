@@ -180,7 +180,10 @@ __global__ __launch_bounds__(kMaxThreads) void svd_jacobi_kernel(
     }
   }
 
-  const T tol2 = (Eps<T>::v * T(n)) * (Eps<T>::v * T(n));
+  // FP32 keeps rotating to 4 units of roundoff (the dot products are good to about one), or the
+  // directions would be off by n of them over the gap of their singular values
+  const T tol = sizeof(T) == 8 ? Eps<T>::v * T(n) : T(4) * Eps<T>::v;
+  const T tol2 = tol * tol;
   // Two rotations side by side, columns (a0, b0) and (a1, b1) with squared norms na, nb.  With
   // zeta = (nb - na) / (2 gamma) = cot(2 theta): r = (1 + zeta^2)^(-1/2), c^2 = (1 + |zeta| r) / 2,
   // s = sign(zeta) r / (2 c), from the reciprocal (square root) instructions as they are, to about
