@@ -19,111 +19,124 @@ namespace isvd {
 
 namespace {
 
-constexpr int kCqThreads = 1024;
-constexpr int kCqGroups = kCqThreads / 128;  // column groups of the trailing update
-constexpr int kCqLanes = kCqThreads / 128;   // lanes per row of the triangular inverse
+constexpr int kCqMax = 1024;  // threads at most: n = 128
+
+// 1/d to rounding: the instruction's approximation and two Newton steps
+__device__ __forceinline__ double rcp_newton(double d) {
+  double w = __builtin_amdgcn_rcp(d);
+  w = w * (2.0 - d * w);
+  return w * (2.0 - d * w);
+}
 
 // One workgroup per l x l block: W (full symmetric storage, upper triangle read) -> R (upper
 // Cholesky factor, W = R^T R, lower part zero) and Rinv = R^-1 (upper).  With check, first
 // ||W - I||_F is formed and more than 1/2 marks the block failed.  status[b] := 1 on failure
 // (non-positive or non-finite pivot); the outputs of a failed block are not used.
-template <typename T>
-__global__ __launch_bounds__(kCqThreads) void chol_inv_kernel(int n, const T *__restrict__ W,
-                                                              T *__restrict__ R,
-                                                              T *__restrict__ Rinv, int check,
-                                                              int *__restrict__ status) {
-  extern __shared__ unsigned char smem_raw[];
-  T *A = reinterpret_cast<T *>(smem_raw);  // n x n, ld n + 1
-  __shared__ T tmp[128];
-  __shared__ T red[kCqThreads];
-  __shared__ int fail;
-  __shared__ T piv;
-  const int b = blockIdx.x, t = threadIdx.x, ld = n + 1;
-  const T *Wb = W + (i64)b * n * n;
-  if (t == 0) fail = 0;
-  T dev = 0;
-  for (int e = t; e < n * n; e += kCqThreads) {
-    const int i = e % n, j = e / n;
-    const T v = (i <= j) ? Wb[i + (i64)j * n] : Wb[j + (i64)i * n];
-    A[i + j * ld] = v;
-    const T d = v - (i == j ? T(1) : T(0));
-    dev += d * d;
-  }
-  red[t] = dev;
-  __syncthreads();
+//
+// The elimination of W = L D L^T and of L X = I in one pass: row i of the working matrix holds
+// W's remaining part in columns > k and X = L^-1 in columns <= k, and step k subtracts l_i = W(i,
+// k) / d_k times row k from every row i > k (X(i, k) := -l_i).  R = D^(1/2) L^T is row k itself
+// over d_k^(1/2), R^-1 = L^-T D^(-1/2) is X^T.  Thread (ti, tj) keeps rows 4 ti .. 4 ti + 3 of
+// columns 4 tj .. 4 tj + 3 in registers, so a step is one barrier, the publishing of one row
+// through LDS and eight reads of it.  One problem (the matrix in LDS, five barriers and a division
+// per column in two passes before): l = 32 40 -> 13.5 us, 48 65 -> 35.5, 64 96 -> 47.3, 128 265 -> 144.
+__global__ __launch_bounds__(kCqMax) void chol_inv_kernel(int n, int n4,
+                                                          const double *__restrict__ W,
+                                                          double *__restrict__ R,
+                                                          double *__restrict__ Rinv, int check,
+                                                          int *__restrict__ status) {
+  __shared__ __align__(16) double row[2][128];
+  __shared__ double dia[128];
+  __shared__ double red[kCqMax / 64];
+  const int b = blockIdx.x, t = threadIdx.x;
+  const double *Wb = W + (i64)b * n * n;
+  double *Rb = R + (i64)b * n * n, *Ib = Rinv + (i64)b * n * n;
+  const bool live = t < n4 * n4;
+  const int ti = live ? t % n4 : 0, tj = live ? t / n4 : 0;
+  const int i0 = 4 * ti, j0 = 4 * tj;
+  double a[4][4];
+  double dev = 0;
+#pragma unroll
+  for (int p = 0; p < 4; ++p)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int i = i0 + p, j = j0 + q;
+      double v = i == j ? 1.0 : 0.0;  // rows and columns past n: the identity
+      if (i < n && j < n) v = (i <= j) ? Wb[i + (i64)j * n] : Wb[j + (i64)i * n];
+      a[p][q] = v;
+      const double d = v - (i == j ? 1.0 : 0.0);
+      if (live) dev += d * d;
+    }
+  bool fail = false;
   if (check) {
-    for (int h = kCqThreads / 2; h > 0; h >>= 1) {
-      if (t < h) red[t] += red[t + h];
-      __syncthreads();
-    }
-    if (t == 0 && !(red[0] <= T(0.25))) fail = 1;  // ||W - I||_F > 1/2, or not finite
+    for (int off = 32; off > 0; off >>= 1) dev += __shfl_xor(dev, off, 64);
+    if ((t & 63) == 0) red[t >> 6] = dev;
+    __syncthreads();
+    double s = 0;
+    for (int w = 0; w < (int)blockDim.x / 64; ++w) s += red[w];
+    if (!(s <= 0.25)) fail = true;  // ||W - I||_F > 1/2, or not finite
   }
-  // right-looking Cholesky of the upper triangle, in place: row k of R at step k
-  for (int k = 0; k < n; ++k) {
-    if (t == 0) {
-      const T d = A[k + k * ld];
-      if (!(d > T(0)) || !(d < T(INFINITY))) fail = 1;
-      A[k + k * ld] = (d > T(0)) ? sqrt(d) : T(1);
-    }
-    __syncthreads();
-    const T rkk = A[k + k * ld];
-    for (int j = k + 1 + t; j < n; j += kCqThreads) A[k + j * ld] /= rkk;
-    __syncthreads();
-    // A(i, j) -= R(k, i) R(k, j) for k < i <= j: a fixed row i per thread, columns strided by
-    // the number of column groups
-    {
-      const int i = k + 1 + (t & 127);
-      if (i < n) {
-        const T rki = A[k + i * ld];
-        for (int j = i + ((t >> 7) + kCqGroups - ((i - k - 1) % kCqGroups)) % kCqGroups; j < n;
-             j += kCqGroups)
-          A[i + j * ld] -= rki * A[k + j * ld];
+  for (int kb = 0; kb < n4; ++kb) {
+#pragma unroll
+    for (int ku = 0; ku < 4; ++ku) {
+      const int k = 4 * kb + ku;
+      double *v = row[ku & 1];
+      if (live && ti == kb) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[j0 + q] = a[ku][q];
+      }
+      __syncthreads();
+      double d = v[k];
+      if (!(d > 0.0) || !(d < (double)INFINITY)) {
+        fail = true;
+        d = 1.0;
+      }
+      if (t == 0) dia[k] = d;
+      const double w = rcp_newton(d);
+      double l[4], c[4];
+#pragma unroll
+      for (int p = 0; p < 4; ++p) l[p] = i0 + p > k ? v[i0 + p] * w : 0.0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) c[q] = v[j0 + q];
+#pragma unroll
+      for (int p = 0; p < 4; ++p)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) a[p][q] -= l[p] * c[q];
+      if (tj == kb) {
+#pragma unroll
+        for (int p = 0; p < 4; ++p) a[p][ku] = i0 + p > k ? -l[p] : a[p][ku];
+      }
+      // row k of R: the published row over d^(1/2) from the diagonal on
+      if (live && ti == kb) {
+        const double s = 1.0 / sqrt(d);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (k < n && j0 + q < n) Rb[k + (i64)(j0 + q) * n] = j0 + q >= k ? c[q] * s : 0.0;
       }
     }
-    __syncthreads();
-  }
-  T *Rb = R + (i64)b * n * n, *Ib = Rinv + (i64)b * n * n;
-  for (int e = t; e < n * n; e += kCqThreads) {
-    const int i = e % n, j = e / n;
-    Rb[i + (i64)j * n] = (i <= j) ? A[i + j * ld] : T(0);
   }
   __syncthreads();
-  // in-place inverse of the upper triangle, column by column (the leading j x j block already
-  // holds its inverse T): x = R(0:j, j);  Rinv(0:j, j) = -T x / R(j, j);  Rinv(j, j) = 1 / R(j, j)
-  // (the pivot is copied in the first phase: thread 0 replaces A(j, j) in the second, where no
-  // other thread reads it)
-  // Each row's sum is split over kCqLanes consecutive lanes (k = i + q, i + q + kCqLanes, ...),
-  // added in a fixed tree.
-  for (int j = 0; j < n; ++j) {
-    for (int i = t; i < j; i += kCqThreads) tmp[i] = A[i + j * ld];
-    if (t == 0) piv = A[j + j * ld];
-    __syncthreads();
-    const T rjj = piv;
-    {
-      const int i = t / kCqLanes, q = t % kCqLanes;
-      T s = 0;
-      if (i < j)
-        for (int k = i + q; k < j; k += kCqLanes) s += A[i + k * ld] * tmp[k];
-      for (int off = kCqLanes / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-      if (i < j && q == 0) A[i + j * ld] = -s / rjj;
+  // R^-1(j, i) = X(i, j) / d_i^(1/2) for j <= i, X(i, i) = 1
+  if (live) {
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const int i = i0 + p;
+      if (i >= n) continue;
+      const double s = 1.0 / sqrt(dia[i]);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int j = j0 + q;
+        if (j < n) Ib[j + (i64)i * n] = j < i ? a[p][q] * s : (j == i ? s : 0.0);
+      }
     }
-    if (t == 0) A[j + j * ld] = T(1) / rjj;
-    __syncthreads();
   }
-  for (int e = t; e < n * n; e += kCqThreads) {
-    const int i = e % n, j = e / n;
-    Ib[i + (i64)j * n] = (i <= j) ? A[i + j * ld] : T(0);
-  }
-  if (t == 0) status[b] = fail;
+  if (t == 0) status[b] = fail ? 1 : 0;
 }
 
-template <typename T>
-void chol_inv(i64 n, i64 batch, const T *W, T *R, T *Rinv, int check, int *status) {
-  const size_t shmem = sizeof(T) * (size_t)n * (size_t)(n + 1);
-  HIP_CHECK(hipFuncSetAttribute((const void *)chol_inv_kernel<T>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem));
-  hipLaunchKernelGGL(chol_inv_kernel<T>, dim3((unsigned)batch), dim3(kCqThreads), shmem,
-                     ctx().stream, (int)n, W, R, Rinv, check, status);
+void chol_inv(i64 n, i64 batch, const double *W, double *R, double *Rinv, int check, int *status) {
+  const int n4 = (int)((n + 3) / 4), nt = (n4 * n4 + 63) / 64 * 64;
+  hipLaunchKernelGGL(chol_inv_kernel, dim3((unsigned)batch), dim3(nt), 0, ctx().stream, (int)n, n4,
+                     W, R, Rinv, check, status);
   LAUNCH_CHECK();
 }
 
@@ -150,7 +163,7 @@ void chol_step(i64 l, i64 batch, const T *w, double *w64, double *r, double *rin
   } else {
     convert<double, float>(l, l * batch, w, l, w64, l);
   }
-  chol_inv<double>(l, batch, wd, r, rinv64, check, status);
+  chol_inv(l, batch, wd, r, rinv64, check, status);
   if constexpr (!std::is_same_v<T, double>) convert<float, double>(l, l * batch, rinv64, l, rinv, l);
 }
 
