@@ -181,18 +181,18 @@ bool cholqr2_rowmajor(i64 m, i64 l, T *Y, i64 ldy, i64 sY, i64 batch, T *R, i64 
   if constexpr (dbl) rinv_data = rinv.get();
   else rinv_data = rinv_t.get();
   // pass 1: W1 = Y^T Y, W1 = R1^T R1, Z^T = R1^-T Y^T
-  gemm<T>('N', 'T', l, l, m, T(1), Y, ldy, Y, ldy, T(0), w.get(), l, batch, sY, sY, ll);
+  gram_rows<T>(l, m, Y, ldy, sY, w.get(), batch);
   chol_step<T>(l, batch, w.get(), w64.get(), r1.get(), rinv.get(), rinv_data, 0, st.get());
-  gemm<T>('T', 'N', l, m, l, T(1), rinv_data, l, Y, ldy, T(0), z.get(), ldz, batch, ll, sY, l);
+  apply_upper<T>(l, m, rinv_data, Y, ldy, sY, z.get(), ldz, l, batch);
   // pass 2 on Z, certified by ||Z^T Z - I||_F <= 1/2
-  gemm<T>('N', 'T', l, l, m, T(1), z.get(), ldz, z.get(), ldz, T(0), w.get(), l, batch, l, l, ll);
+  gram_rows<T>(l, m, z.get(), ldz, l, w.get(), batch);
   chol_step<T>(l, batch, w.get(), w64.get(), r2.get(), rinv.get(), rinv_data, 1,
                st.get() + batch);
   std::vector<int> h(2 * batch);
   read_back(h.data(), st.get(), sizeof(int) * 2 * batch);
   for (int v : h)
     if (v) return false;
-  gemm<T>('T', 'N', l, m, l, T(1), rinv_data, l, z.get(), ldz, T(0), Y, ldy, batch, ll, l, sY);
+  apply_upper<T>(l, m, rinv_data, z.get(), ldz, l, Y, ldy, sY, batch);
   // R = R2 R1
   if (R) {
     if constexpr (dbl) {

@@ -43,6 +43,16 @@ void gemm_ct(char transa, char transb, i64 m, i64 n, i64 k, T alpha, const T *A,
 template <typename T>
 void syrk_full(char trans, i64 n, i64 k, T alpha, const T *A, i64 lda, T *C, i64 ldc);
 
+// W_b := Y_b^T Y_b (l x l, dense) for `batch` row-major m x l blocks Y_b = Y + b sY, row stride ldy.
+template <typename T>
+void gram_rows(i64 l, i64 m, const T *Y, i64 ldy, i64 sY, T *W, i64 batch);
+
+// Z_b := Y_b X_b for the same blocks and upper triangular X_b (l x l, dense column-major; its
+// lower part must be zero), Z_b = Z + b sZ row-major with row stride ldz, apart from Y.
+template <typename T>
+void apply_upper(i64 l, i64 m, const T *X, const T *Y, i64 ldy, i64 sY, T *Z, i64 ldz, i64 sZ,
+                 i64 batch);
+
 // B := alpha * op(A)   (m x n result; mkl_?omatcopy semantics, 'N' or 'T').
 template <typename T>
 void omatcopy(char trans, i64 m, i64 n, T alpha, const T *A, i64 lda, T *B, i64 ldb,

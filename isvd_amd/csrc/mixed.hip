@@ -73,7 +73,7 @@ void stage_orth_gramian_b(const Dims &d, float *yst, i64 ldyst, bool cholqr) {
     float *dst = pass == 0 ? other.get() : yst;
     const i64 ldd = pass == 0 ? Nl : ldyst;
     // W_i := Y_i^T Y_i
-    gemm<float>('N', 'T', l, l, m, 1.f, src, lds, src, lds, 0.f, w32.get(), l, N, l, l, l * l);
+    gram_rows<float>(l, m, src, lds, l, w32.get(), N);
     convert<double, float>(l, l * N, w32.get(), l, w64.get(), l);
     // W_i = U_i diag(s_i) U_i^T; U_i := U_i diag(s_i)^{-1/2}
     eig_psd_small<double>(l, w64.get(), l, l * l, s64.get(), l, u64.get(), l, l * l, N);

@@ -275,7 +275,7 @@ void stage_orth_gramian(const Dims &d, T *yst, i64 ldyst, bool cholqr) {
   const i64 l = d.l, N = d.N, m = d.m;
   DBuf<T> w(l * d.Nl), u(l * d.Nl), s(l * N), ycopy(ldyst * m);
   // W_i := Y_i^T Y_i  (:81-84)
-  gemm<T>('N', 'T', l, l, m, T(1), yst, ldyst, yst, ldyst, T(0), w.get(), l, N, l, l, l * l);
+  gram_rows<T>(l, m, yst, ldyst, l, w.get(), N);
   // gesvd('O','N') of every W_i  (:87-90)
   eig_psd_small<T>(l, w.get(), l, l * l, s.get(), l, u.get(), l, l * l, N);
   // s := sqrt(s); U_i := U_i / s_i  (:91, :94)
@@ -793,7 +793,7 @@ void post_gramian_z(const Dims &d, const T *qt, i64 ldqt, T *zt, T *s, T *ut, i6
   const i64 l = d.l, k = d.k;
   DBuf<T> w(l * l), uw(l * l);
   // W := Z^T Z (:145); gesvd('O','N') + vSqrt (:149-151)
-  gemm<T>('N', 'T', l, l, d.n, T(1), zt, l, zt, l, T(0), w.get(), l);
+  gram_rows<T>(l, d.n, zt, l, 0, w.get(), 1);
   eig_psd_small<T>(l, w.get(), l, 0, s, l, uw.get(), l, 0, 1);
   hipLaunchKernelGGL(sqrt_inplace_kernel<T>, dim3(1, 1), dim3(256), 0, ctx().stream, (int)l, s);
   LAUNCH_CHECK();
