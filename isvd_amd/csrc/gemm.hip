@@ -6,9 +6,10 @@
 // walk the contiguous dimension of each operand, so both the "N" and the "T" forms load
 // coalesced.  A register-prefetch double buffer overlaps the next tile's global loads with
 // the current tile's MFMAs (one barrier per K tile).
-// The large FP64 products (128 x 256 tiles) run instead on gemm_dl_kernel, which fills LDS
-// straight from global memory three K steps ahead; the register-staged kernel keeps the
-// smaller tiles, FP32, and operands that are not 16-byte aligned.
+// Large products with a row-contiguous op(A) run instead on gemm_stream_kernel, which takes no
+// LDS; those with a K-contiguous one on gemm_dl_kernel / gemm_dl32_kernel (128 x 256 tiles), which
+// fill LDS straight from global memory three K steps ahead.  The register-staged kernel keeps the
+// smaller tiles and the operands that gemm_dl_kernel's alignment rules exclude.
 #include "la.hpp"
 #include "lds_dma.hpp"
 #include "mfma.hpp"
@@ -266,32 +267,32 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_kernel(GemmArgs<T> g) {
 // (global_load_lds_dwordx4, no register staging), three K steps in flight.
 //
 // Tile 128 x 256 x 16, eight waves in a 2 x 4 grid of 64 x 64 (4 x 4 fragments of
-// v_mfma_f64_16x16x4f64).  Each operand tile has one of two LDS layouts, chosen by which of
-// its dimensions is contiguous in global memory:
+// v_mfma_f64_16x16x4f64).  op(B) = B is K-contiguous; op(A) may be either.  An operand tile's LDS
+// layout follows which of its dimensions is contiguous in global memory:
 //   K-contiguous (op(A) = A^T, op(B) = B): one 128-byte row of 16 K values per tile row; the
 //     eight 16-byte chunks of row r sit at position chunk ^ ((r >> 1) & 7), so that the
 //     16 rows of a fragment read fall in distinct banks.  A fill instruction covers 8 rows:
 //     lane l fetches row 8 j + l / 8, chunk (l % 8) ^ swizzle (the LDS position is fixed to
 //     l % 8 by the instruction).
-//   MN-contiguous (op(A) = A, op(B) = B^T): one K row of the tile per 1 KB (A) or 2 KB (B),
-//     padded by 64 bytes so that rows 2 apart start 128 bytes apart in the banks.
+//   M-contiguous (op(A) = A): one K row of the tile per 1 KB, padded by 64 bytes so that rows 2
+//     apart start 128 bytes apart in the banks.
 // The MFMA consumes K in pairs: lane l / 16 = s supplies K index k8 + 2 s + h to the
 // instruction h of a pair (h = 0, 1), so a K-contiguous fragment is one 16-byte LDS read
 // serving both instructions, and the two operands agree on the K index of every product.
 // Rows past the matrix edge are fetched from the last valid row (or column pair): they feed
 // only outputs that are not stored.  Requirements (checked by the host): 16-byte aligned
-// operands, even leading dimensions and batch strides, even m (n) when op(A) (op(B)) is
-// MN-contiguous.  A partial last K step goes through registers with bounds checks.
+// operands, even leading dimensions and batch strides, even m when op(A) is M-contiguous.  A
+// partial last K step goes through registers with bounds checks.
 namespace dl {
 constexpr int BM = 128, BN = 256, BK = 16, NT = 512, S = 3;
-constexpr int PITCH_A = BM * 8 + 64, PITCH_B = BN * 8 + 64;
+constexpr int PITCH_A = BM * 8 + 64;
 constexpr int FILLS = (BM + BN) * BK * 8 / 1024 / (NT / 64);  // per wave per K step
 constexpr int A_FILLS = BM * BK * 8 / 1024;                   // fill instructions for op(A)
 static_assert(A_FILLS % (NT / 64) == 0, "op(A) fills must be whole per-wave slots");
-template <bool KA, bool KB>
+template <bool KA>
 struct Layout {
   static constexpr int A_BYTES = KA ? BM * BK * 8 : BK * PITCH_A;
-  static constexpr int B_BYTES = KB ? BN * BK * 8 : BK * PITCH_B;
+  static constexpr int B_BYTES = BN * BK * 8;
   static constexpr int STAGE = A_BYTES + B_BYTES;
   static_assert(S * STAGE <= 160 * 1024, "LDS budget");
 };
@@ -300,10 +301,10 @@ __device__ inline int swz(int r) { return (r >> 1) & 7; }
 
 typedef double d2 __attribute__((ext_vector_type(2)));
 
-template <bool KA, bool KB>
+template <bool KA>
 __global__ __launch_bounds__(dl::NT) void gemm_dl_kernel(GemmArgs<double> g) {
   using namespace dl;
-  using L = Layout<KA, KB>;
+  using L = Layout<KA>;
   // one LDS object per stage: the compiler then sees that a fill of one stage and the
   // fragment reads of another do not alias
   __shared__ __align__(16) unsigned char st0[L::STAGE], st1[L::STAGE], st2[L::STAGE];
@@ -332,7 +333,7 @@ __global__ __launch_bounds__(dl::NT) void gemm_dl_kernel(GemmArgs<double> g) {
   // wave-uniform operand bases at this chunk's first K step; per lane, a 32-bit element
   // offset for each fill slot (the host keeps the leading dimensions below 2^23)
   const double *abase = Ab + (KA ? m0 * g.lda + kbeg : m0 + kbeg * g.lda);
-  const double *bbase = Bb + (KB ? n0 * g.ldb + kbeg : n0 + kbeg * g.ldb);
+  const double *bbase = Bb + n0 * g.ldb + kbeg;
   unsigned off[FILLS], loff[FILLS];
 #pragma unroll
   for (int u = 0; u < FILLS; ++u) {
@@ -350,21 +351,13 @@ __global__ __launch_bounds__(dl::NT) void gemm_dl_kernel(GemmArgs<double> g) {
       }
     } else {
       const int fb = f - A_FILLS;
-      if (KB) {
-        const int row = 8 * fb + (lane >> 3), c = (lane & 7) ^ swz(row);
-        const i64 gj = (n0 + row < g.n) ? row : g.n - 1 - n0;
-        off[u] = (unsigned)(gj * g.ldb + 2 * c);
-        loff[u] = L::A_BYTES + fb * 1024;
-      } else {
-        const int q = fb >> 1, h = fb & 1;
-        const i64 j =
-            (n0 + 128 * h + 2 * lane <= g.n - 2) ? 128 * h + 2 * lane : g.n - 2 - n0;
-        off[u] = (unsigned)(j + q * g.ldb);
-        loff[u] = L::A_BYTES + q * PITCH_B + h * 1024;
-      }
+      const int row = 8 * fb + (lane >> 3), c = (lane & 7) ^ swz(row);
+      const i64 gj = (n0 + row < g.n) ? row : g.n - 1 - n0;
+      off[u] = (unsigned)(gj * g.ldb + 2 * c);
+      loff[u] = L::A_BYTES + fb * 1024;
     }
   }
-  const i64 dA = KA ? BK : BK * g.lda, dB = KB ? BK : BK * g.ldb;  // per K step
+  const i64 dA = KA ? BK : BK * g.lda, dB = BK;  // per K step
   auto fill = [&](i64 kt, unsigned char *st) {
     const unsigned base = lds_addr(st);
     const double *ak = abase + kt * dA, *bk = bbase + kt * dB;
@@ -378,8 +371,7 @@ __global__ __launch_bounds__(dl::NT) void gemm_dl_kernel(GemmArgs<double> g) {
     return KA ? row * 128 + (((k >> 1) ^ swz(row)) << 4) + (k & 1) * 8 : k * PITCH_A + row * 8;
   };
   auto b_off = [](int col, int k) {
-    return L::A_BYTES +
-           (KB ? col * 128 + (((k >> 1) ^ swz(col)) << 4) + (k & 1) * 8 : k * PITCH_B + col * 8);
+    return L::A_BYTES + col * 128 + (((k >> 1) ^ swz(col)) << 4) + (k & 1) * 8;
   };
   // the partial last K step: registers with bounds checks, zeros past kend
   auto fill_checked = [&](i64 k0, unsigned char *st) {
@@ -391,10 +383,10 @@ __global__ __launch_bounds__(dl::NT) void gemm_dl_kernel(GemmArgs<double> g) {
       *reinterpret_cast<double *>(st + a_off(row, k)) = v;
     }
     for (int e = t; e < BN * BK; e += NT) {
-      const int col = KB ? e >> 4 : e % BN, k = KB ? e & 15 : e / BN;
+      const int col = e >> 4, k = e & 15;
       const i64 gj = n0 + col, gk = k0 + k;
       double v = 0.0;
-      if (gj < g.n && gk < kend) v = KB ? Bb[gk + gj * g.ldb] : Bb[gj + gk * g.ldb];
+      if (gj < g.n && gk < kend) v = Bb[gk + gj * g.ldb];
       *reinterpret_cast<double *>(st + b_off(col, k)) = v;
     }
   };
@@ -425,14 +417,9 @@ __global__ __launch_bounds__(dl::NT) void gemm_dl_kernel(GemmArgs<double> g) {
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
       const int c = wn * 64 + 16 * b + lr;
-      if (KB) {
-        const d2 v = *reinterpret_cast<const d2 *>(st + b_off(c, k));
-        fb[b][0] = v.x;
-        fb[b][1] = v.y;
-      } else {
-        fb[b][0] = *reinterpret_cast<const double *>(st + b_off(c, k));
-        fb[b][1] = *reinterpret_cast<const double *>(st + b_off(c, k + 1));
-      }
+      const d2 v = *reinterpret_cast<const d2 *>(st + b_off(c, k));
+      fb[b][0] = v.x;
+      fb[b][1] = v.y;
     }
   };
   // the 16 products of instruction h of a half step
@@ -516,7 +503,7 @@ typedef float f4v __attribute__((ext_vector_type(4)));
 
 __global__ __launch_bounds__(dl::NT) void gemm_dl32_kernel(GemmArgs<float> g) {
   using namespace dl;
-  using L = Layout<true, true>;  // 128-byte rows for both operands, as in the FP64 kernel
+  using L = Layout<true>;  // 128-byte rows for both operands, as in the FP64 kernel
   static_assert(L::A_BYTES == BM * BK32 * 4 && L::B_BYTES == BN * BK32 * 4, "row layout");
   __shared__ __align__(16) unsigned char st0[L::STAGE], st1[L::STAGE], st2[L::STAGE];
   auto stage = [&](auto k) -> unsigned char * {
@@ -652,15 +639,14 @@ inline bool dl32_eligible(const GemmArgs<float> &g, i64 batch) {
   return true;
 }
 
-// Whether gemm_dl_kernel<KA, KB> can take this product (every fill is an aligned 16-byte
+// Whether gemm_dl_kernel<KA> can take this product (every fill is an aligned 16-byte
 // read inside the operands).
-inline bool dl_eligible(const GemmArgs<double> &g, bool KA, bool KB, i64 batch) {
+inline bool dl_eligible(const GemmArgs<double> &g, bool KA, i64 batch) {
   auto aligned = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
   if (!aligned(g.A) || !aligned(g.B)) return false;
   if ((g.lda & 1) || (g.ldb & 1)) return false;
   if (batch > 1 && ((g.sA & 1) || (g.sB & 1))) return false;
   if (!KA && (g.m & 1)) return false;
-  if (!KB && (g.n & 1)) return false;
   // per-lane fill offsets are 32-bit element counts below 256 leading dimensions
   if (g.lda >= (1 << 23) || g.ldb >= (1 << 23)) return false;
   return true;
@@ -668,7 +654,7 @@ inline bool dl_eligible(const GemmArgs<double> &g, bool KA, bool KB, i64 batch) 
 
 }  // namespace isvd
 
-#include "gemm_thin.hpp"
+#include "gemm_stream.hpp"
 
 namespace isvd {
 
@@ -796,10 +782,10 @@ void launch_cfg(GemmArgs<T> g, i64 batch) {
   ISVD_CHECK(batch * ksplit <= 65535, "grid.y too large (batch %lld x ksplit %d)", batch, ksplit);
   dim3 grid((unsigned)tiles, (unsigned)(batch * ksplit));
   bool done = false;
-  // (op(A) = A^T with op(B) = B^T, unused by the stages, stays on the register-staged kernel)
-  if constexpr (std::is_same_v<T, double> && BM == dl::BM && BN == dl::BN && !(TA && TB)) {
-    if (dl_eligible(g, TA, !TB, batch)) {
-      hipLaunchKernelGGL((gemm_dl_kernel<TA, !TB>), grid, dim3(dl::NT), 0, ctx().stream, g);
+  // (op(B) = B^T with a tile this large is gemm_stream_kernel's, or small, or not used by the stages)
+  if constexpr (std::is_same_v<T, double> && BM == dl::BM && BN == dl::BN && !TB) {
+    if (dl_eligible(g, TA, batch)) {
+      hipLaunchKernelGGL((gemm_dl_kernel<TA>), grid, dim3(dl::NT), 0, ctx().stream, g);
       done = true;
     }
   }
@@ -849,43 +835,115 @@ int fixed64(char transa, char transb, GemmArgs<T> g, i64 batch, int ksplit) {
   return launch_fixed64<T, true, true>(g, batch, ksplit);
 }
 
-// Few rows against a large op(B): gemm_thin_kernel, from K = 1024 and n = 256 on (below, a product
-// is a few microseconds either way).  FP32 with more than 48 rows only from 2^26 elements of B on:
-// a 3001 x 8191 B with unaligned columns takes 73 us against 69 us on 64 x 64 tiles there (59 / 68
-// at 48 rows; FP64 83 / 106 at 64).
+// How gemm_stream_kernel takes a product: MT row tiles and E strips per wave, ks chunks of K.
+struct StreamPlan {
+  int MT = 0, E = 1;
+  i64 ks = 1, blocks = 0;
+};
+
+// Workgroups of one K chunk.
 template <typename T>
-bool thin_eligible(const GemmArgs<T> &g, i64 batch) {
-  if (g.ct || g.upper || g.m > 64 || g.n < 256 || g.k < 1024 || batch > 1024) return false;
-  return sizeof(T) == 8 || g.m <= 48 || g.n * g.k >= (1ll << 26);
+i64 stream_blocks(const GemmArgs<T> &g, int MT, int E) {
+  const i64 rows = 16 * MT, cols = stream::Traits<T>::COLS * E;
+  const i64 rblocks = (g.m + rows - 1) / rows, strips = (g.n + cols - 1) / cols;
+  if (!g.upper) return rblocks * strips;
+  i64 total = 0;
+  for (i64 q = 0; q < strips; ++q) total += stream::upper_blocks(q, rows, cols, rblocks);
+  return total;
+}
+
+template <typename T>
+StreamPlan stream_plan(const GemmArgs<T> &g, bool KB, i64 batch) {
+  using X = stream::Traits<T>;
+  StreamPlan p;
+  if (g.ct || batch > 1024) return p;
+  // per-lane offsets are 32-bit byte counts below 16 * 8 leading dimensions
+  if (g.lda >= (1 << 22) || g.ldb >= (1 << 22)) return p;
+  const i64 min_chunk = 16 * X::STEP;
+  if (g.m <= 64) {
+    // Few rows against a large op(B), from K = 1024 and n = 256 on (below, a product is a few
+    // microseconds either way).  FP32 with more than 48 rows only from 2^26 elements of B on: a
+    // 3001 x 8191 B with unaligned columns takes 73 us against 69 us on 64 x 64 tiles there (59 / 68
+    // at 48 rows; FP64 83 / 106 at 64).
+    if (g.upper || g.n < 256 || g.k < 1024) return p;
+    if (sizeof(T) == 4 && g.m > 48 && g.n * g.k < (1ll << 26)) return p;
+    p.MT = (int)((g.m + 15) / 16);
+    p.blocks = stream_blocks(g, p.MT, 1);
+    // one workgroup per CU, and partial sums (written and read) below half of B's bytes
+    i64 ks = (256 + p.blocks * batch - 1) / (p.blocks * batch);
+    const i64 by_k = g.k / min_chunk, by_bytes = g.k / (4 * g.m);
+    if (ks > by_k) ks = by_k;
+    if (ks > by_bytes) ks = by_bytes;
+    p.ks = ks < 1 ? 1 : ks;
+    return p;
+  }
+  // More rows.  FP64 from 3 * 2^24 products on (1000 x 512 x 80: 37 against 35 us; 200 x 4096 x 65: 44
+  // against 52), FP32, whose workgroup of 64 x 512 on a CU of its own wants a large product, from
+  // 2^33 and K = 1024 on (4001 x 1000 x 512: 109 against 91 us, 20000 x 4096 x 128: 241 / 259).
+  const double mnk = (double)g.m * (double)g.n * (double)g.k;
+  constexpr bool dbl = sizeof(T) == 8;
+  if (g.n < 64 || g.k < 64) return p;
+  if (dbl ? mnk < 3.0 * (1 << 24) : (g.k < 1024 || mnk < (double)(1ll << 33))) return p;
+  // One row tile of gemm_dl_kernel reads a K-contiguous B once where two blocks of 64 rows read it
+  // twice, which shows where its columns are far apart: 128 rows, 16384 columns of 131072 values 8.18
+  // against 7.86 ms, of 32768 2.04 / 2.02, of 16384 1.03 / 1.04 (100 rows, of 131072: 7.9 / 12.3).
+  if constexpr (dbl)
+    if (KB && g.m > 112 && g.m <= 128 && g.k >= (1 << 15) && dl_eligible(g, false, batch)) return p;
+  // The split that the busiest CU is done with first: its share of the blocks at the rate of a full
+  // CU (74 and 134 TFLOP/s on the card), what a block costs beside its products (one FP32 workgroup
+  // fills a CU: nothing runs beside its first loads and its stores, 20 us), and the partial sums'
+  // way through memory.
+  const i64 cus = ctx().max_wgs > 0 ? ctx().max_wgs : ctx().cus;
+  // FP64 strips of 64 columns a wave from 2^35 products on (32768 x 16384 x 4096: 59.7 against 62.5
+  // ms; 60000 x 4001 x 128: 1064 / 1131 us), of 32 below (4096 x 4096 x 512: 288 / 271 us)
+  const bool wide = !dbl || mnk >= (double)(1ll << 35);
+  double best = 1e30;
+  for (int MT = 4; MT >= 3; --MT) {
+    const int E = wide ? 2 : 1;
+    const i64 blocks = stream_blocks(g, MT, E);
+    const double tile = 2.0 * 16 * MT * X::COLS * E * (MT == 4 ? 1.0 : 1.03) / (dbl ? 0.29e12 : 0.52e12);
+    for (i64 ks = 1; ks <= 64; ++ks) {
+      const i64 chunk = (g.k + ks - 1) / ks, share = (blocks * batch * ks + cus - 1) / cus;
+      if (ks > 1 && chunk < min_chunk) break;
+      double t = (double)share * (tile * (double)chunk + (dbl ? 2e-6 : 20e-6));
+      if (ks > 1) t += (double)(ks + 1) * 2 * sizeof(T) * (double)(g.m * g.n * batch) / 8e12 + 3e-6;
+      if (t < 0.98 * best) {
+        best = t;
+        p.MT = MT; p.E = E; p.ks = ks; p.blocks = blocks;
+      }
+    }
+  }
+  return p;
 }
 
 template <typename T, bool KB>
-void launch_thin(GemmArgs<T> g, i64 batch) {
-  using X = thin::Traits<T>;
-  const i64 blocks = (g.n + X::COLS - 1) / X::COLS;
-  // one workgroup per CU; a chunk of at least 8 groups of steps, and partial sums (written and
-  // read) below half of B's bytes
-  i64 ks = (256 + blocks * batch - 1) / (blocks * batch);
-  const i64 by_k = g.k / (8 * X::U * X::STEP), by_bytes = g.k / (4 * g.m);
-  if (ks > by_k) ks = by_k;
-  if (ks > by_bytes) ks = by_bytes;
+void launch_stream(GemmArgs<T> g, const StreamPlan &p, i64 batch) {
+  using X = stream::Traits<T>;
+  i64 ks = p.ks;
   if (ctx().max_wgs > 0)
-    while (ks > 1 && blocks * batch * ks > ctx().max_wgs) --ks;
+    while (ks > 1 && p.blocks * batch * ks > ctx().max_wgs) --ks;
   const size_t per = sizeof(T) * (size_t)(batch * g.m * g.n);
   while (ks > 1 && per * (size_t)ks > splitk_budget()) --ks;
-  if (ks < 1) ks = 1;
   i64 kchunk = (g.k + ks - 1) / ks;
   kchunk = (kchunk + X::STEP - 1) / X::STEP * X::STEP;
   ks = (g.k + kchunk - 1) / kchunk;
   g.ksplit = (int)ks;
   g.kchunk = kchunk;
+  g.group_m = 16;
   if (ks > 1) g.W = static_cast<T *>(splitk_workspace(per * (size_t)ks));
-  const dim3 grid((unsigned)blocks, (unsigned)(batch * ks));
-  const int mt = (int)((g.m + 15) / 16);
-  if (mt == 1) hipLaunchKernelGGL((gemm_thin_kernel<T, KB, 1>), grid, dim3(thin::NT), 0, ctx().stream, g);
-  else if (mt == 2) hipLaunchKernelGGL((gemm_thin_kernel<T, KB, 2>), grid, dim3(thin::NT), 0, ctx().stream, g);
-  else if (mt == 3) hipLaunchKernelGGL((gemm_thin_kernel<T, KB, 3>), grid, dim3(thin::NT), 0, ctx().stream, g);
-  else hipLaunchKernelGGL((gemm_thin_kernel<T, KB, 4>), grid, dim3(thin::NT), 0, ctx().stream, g);
+  const dim3 grid((unsigned)p.blocks, (unsigned)(batch * ks));
+  auto go = [&](auto mt, auto e) {
+    hipLaunchKernelGGL((gemm_stream_kernel<T, KB, decltype(mt)::value, decltype(e)::value>), grid,
+                       dim3(stream::NT), 0, ctx().stream, g);
+  };
+  using one = std::integral_constant<int, 1>;
+  using two = std::integral_constant<int, 2>;
+  if (p.E == 2 && p.MT == 3) go(std::integral_constant<int, 3>{}, two{});
+  else if (p.E == 2) go(std::integral_constant<int, 4>{}, two{});
+  else if (p.MT == 1) go(one{}, one{});
+  else if (p.MT == 2) go(two{}, one{});
+  else if (p.MT == 3) go(std::integral_constant<int, 3>{}, one{});
+  else go(std::integral_constant<int, 4>{}, one{});
   LAUNCH_CHECK();
   if (ks > 1) splitk_reduce(g, batch);
 }
@@ -893,8 +951,9 @@ void launch_thin(GemmArgs<T> g, i64 batch) {
 template <typename T, bool TA, bool TB>
 void launch(GemmArgs<T> g, i64 batch) {
   if constexpr (!TA) {
-    if (thin_eligible(g, batch)) {
-      launch_thin<T, !TB>(g, batch);
+    const StreamPlan p = stream_plan(g, !TB, batch);
+    if (p.MT > 0) {
+      launch_stream<T, !TB>(g, p, batch);
       return;
     }
   }
