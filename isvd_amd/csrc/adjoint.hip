@@ -147,14 +147,16 @@ __global__ __launch_bounds__(kNormThreads) void rownorm2_parts_kernel(int k, i64
   }
 }
 
+// out[i] := the sum of row i's chunks, one wave per row (one thread per row waited for 128 loads in
+// turn: 19.6 -> 5.1 us)
 template <typename T>
-__global__ __launch_bounds__(128) void rownorm2_final_kernel(int k, int nchunks, const T *part,
-                                                             T *out) {
-  const int i = threadIdx.x;
-  if (i >= k) return;
+__global__ __launch_bounds__(64) void rownorm2_final_kernel(int k, int nchunks, const T *part,
+                                                            T *out) {
+  const int i = blockIdx.x, t = threadIdx.x;
   T r = 0;
-  for (int b = 0; b < nchunks; ++b) r += part[(i64)b * k + i];
-  out[i] = r;
+  for (int b = t; b < nchunks; b += 64) r += part[(i64)b * k + i];
+  for (int off = 32; off; off >>= 1) r += __shfl_xor(r, off);
+  if (t == 0) out[i] = r;
 }
 
 template <typename T>
@@ -165,7 +167,7 @@ void rownorm2(int k, i64 cols, const T *P, i64 ldp, T *out, T *part) {
   hipLaunchKernelGGL(rownorm2_parts_kernel<T>, dim3((unsigned)(nchunks > 0 ? nchunks : 1)),
                      dim3(kNormThreads), 0, ctx().stream, k, cols, chunk, P, ldp, part);
   LAUNCH_CHECK();
-  hipLaunchKernelGGL(rownorm2_final_kernel<T>, dim3(1), dim3(128), 0, ctx().stream, k,
+  hipLaunchKernelGGL(rownorm2_final_kernel<T>, dim3((unsigned)k), dim3(64), 0, ctx().stream, k,
                      nchunks > 0 ? nchunks : 1, (const T *)part, out);
   LAUNCH_CHECK();
 }

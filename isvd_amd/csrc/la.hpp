@@ -17,6 +17,12 @@ void gemm(char transa, char transb, i64 m, i64 n, i64 k, T alpha, const T *A, i6
           const T *B, i64 ldb, T beta, T *C, i64 ldc, i64 batch = 1, i64 sA = 0, i64 sB = 0,
           i64 sC = 0);
 
+// The same product (one problem) always on the LDS-tiled kernels, so that its order of summation does
+// not move with the kernels large products take.
+template <typename T>
+void gemm_tiled(char transa, char transb, i64 m, i64 n, i64 k, T alpha, const T *A, i64 lda,
+                const T *B, i64 ldb, T beta, T *C, i64 ldc);
+
 // The same product on 64 x 64 tiles without split-K: for a short K (<= a few hundred) whose
 // output alone fills the device, where a split would only add a reduction pass.
 template <typename T>
@@ -46,6 +52,12 @@ void syrk_full(char trans, i64 n, i64 k, T alpha, const T *A, i64 lda, T *C, i64
 // W_b := Y_b^T Y_b (l x l, dense) for `batch` row-major m x l blocks Y_b = Y + b sY, row stride ldy.
 template <typename T>
 void gram_rows(i64 l, i64 m, const T *Y, i64 ldy, i64 sY, T *W, i64 batch);
+
+// W_b := alpha X_b^T Y_b + beta W_b (r x l, r and l <= 128) for row-major m x r and m x l blocks;
+// false (nothing done) where it does not apply: larger blocks, no room for its partial sums.
+template <typename T>
+bool cross_rows(i64 r, i64 l, i64 m, T alpha, const T *X, i64 ldx, i64 sX, const T *Y, i64 ldy,
+                i64 sY, T beta, T *W, i64 ldw, i64 sW, i64 batch);
 
 // Z_b := Y_b X_b for the same blocks and upper triangular X_b (l x l, dense column-major; its
 // lower part must be zero), Z_b = Z + b sZ row-major with row stride ldz, apart from Y.

@@ -607,7 +607,9 @@ void stage_integrate_kn(const Dims &d, const KnArgs &args, const T *yst, i64 ldy
 
 // Wen-Yin integration (@x@_integrate_wen_yin.c:201-384), same coordinates as KN:
 // Q_c = Qs xq, G_c = Qs gq (gq = B_c / N), X_c = Qs xx, <Qs a, Qs b> = <a, M b>; the
-// 2l x 2l inverse of the line search is replaced by its closed form (sym_scale_kernel).
+// 2l x 2l inverse of the line search is replaced by its closed form (sym_scale_kernel).  The
+// nonmonotone line search amplifies rounding-level changes into other stopping points, so the updates
+// stay on the tiled product (gemm_tiled) and its order of summation.
 template <typename T>
 void integrate_wy_coords(const Dims &d, const WyArgs &args, const T *M, T *x_out, i64 *iter_out,
                          double *mu_out) {
@@ -628,7 +630,7 @@ void integrate_wy_coords(const Dims &d, const WyArgs &args, const T *M, T *x_out
   gemm_ct<T>('T', 'N', l, Nl, Nl, T(1), gq.get(), Nl, M, Nl, T(0), bgc.get(), Nl);
   gemm<T>('T', 'N', l, l, Nl, ninv, bc.get(), Nl, bgc.get(), Nl, T(0), dgc.get(), l);
   omatcopy<T>('N', Nl, l, T(1), gq.get(), Nl, xx.get(), Nl);
-  gemm<T>('N', 'N', Nl, l, l, T(-1), xq.get(), Nl, dc.get(), l, T(1), xx.get(), Nl);
+  gemm_tiled<T>('N', 'N', Nl, l, l, T(-1), xq.get(), Nl, dc.get(), l, T(1), xx.get(), Nl);
   hipLaunchKernelGGL(wy_mu_kernel<T>, dim3(1), dim3(256), 0, ctx().stream, (int)l,
                      (const T *)dgc.get(), (const T *)dc.get(), scal.get());
   LAUNCH_CHECK();
@@ -661,8 +663,8 @@ void integrate_wy_coords(const Dims &d, const WyArgs &args, const T *M, T *x_out
                          (int)l, fc, (const T *)si.get(), T(-4) * it_ * it_, T(0));
       LAUNCH_CHECK();
       // B+ := Bc Fc + Bgc Fgc  (:270-271)
-      gemm<T>('N', 'N', Nl, l, l, T(1), bc.get(), Nl, fc, l, T(0), bp.get(), Nl);
-      gemm<T>('N', 'N', Nl, l, l, T(1), bgc.get(), Nl, fgc, l, T(1), bp.get(), Nl);
+      gemm_tiled<T>('N', 'N', Nl, l, l, T(1), bc.get(), Nl, fc, l, T(0), bp.get(), Nl);
+      gemm_tiled<T>('N', 'N', Nl, l, l, T(1), bgc.get(), Nl, fgc, l, T(1), bp.get(), Nl);
       dot<T>(Nl * l, bp.get(), bp.get(), scal.get() + 2);
       T hv[2];
       read_back(hv, scal.get() + 2, sizeof(hv));
@@ -679,8 +681,8 @@ void integrate_wy_coords(const Dims &d, const WyArgs &args, const T *M, T *x_out
     phi = (args.eta * zeta * phi + phit) / (args.eta * zeta + 1);
     zeta = args.eta * zeta + 1;
     // Q+ := Qc Fc + Gc Fgc  (:291-292)
-    gemm<T>('N', 'N', Nl, l, l, T(1), xq.get(), Nl, fc, l, T(0), xqp.get(), Nl);
-    gemm<T>('N', 'N', Nl, l, l, T(1), gq.get(), Nl, fgc, l, T(1), xqp.get(), Nl);
+    gemm_tiled<T>('N', 'N', Nl, l, l, T(1), xq.get(), Nl, fc, l, T(0), xqp.get(), Nl);
+    gemm_tiled<T>('N', 'N', Nl, l, l, T(1), gq.get(), Nl, fgc, l, T(1), xqp.get(), Nl);
     // D+ := B+^T B+ / N (:295); G+ := Qs B+ / N (:298); Bg+ := Qs^T G+ (:301-303)
     gemm<T>('T', 'N', l, l, Nl, ninv, bp.get(), Nl, bp.get(), Nl, T(0), dc.get(), l);
     omatcopy<T>('N', Nl, l, ninv, bp.get(), Nl, gq.get(), Nl);
@@ -693,7 +695,7 @@ void integrate_wy_coords(const Dims &d, const WyArgs &args, const T *M, T *x_out
     // X+ := G+ - Q+ D+ (:324-325); Delta1, Delta2 (:328-329), queued before mu is read back so
     // that mu and t come back together (after the last iteration they go unused)
     omatcopy<T>('N', Nl, l, T(1), gq.get(), Nl, xxp.get(), Nl);
-    gemm<T>('N', 'N', Nl, l, l, T(-1), xqp.get(), Nl, dc.get(), l, T(1), xxp.get(), Nl);
+    gemm_tiled<T>('N', 'N', Nl, l, l, T(-1), xqp.get(), Nl, dc.get(), l, T(1), xxp.get(), Nl);
     hipLaunchKernelGGL(sub_kernel<T>, dim3(grid_for(Nl * l)), dim3(256), 0, ctx().stream,
                        Nl * l, (const T *)xq.get(), (const T *)xqp.get(), d1.get());
     hipLaunchKernelGGL(sub_kernel<T>, dim3(grid_for(Nl * l)), dim3(256), 0, ctx().stream,
