@@ -64,6 +64,8 @@ struct BgArgs {
   i64 kchunk;       // K values per chunk (multiple of BK)
   float *W;         // split-K partials: [ksplit][N][M]
   i64 upper_rows;   // tiles inside rows 0 .. upper_rows-1 strictly below the diagonal are skipped
+  i64 tile0, ntiles;  // the launch computes tiles tile0 .. tile0 + ntiles - 1 of the raster
+  int tail;         // 1: K chunks of single tiles, partials in W as [tile][chunk][256 x 256]
 };
 
 namespace bg {
@@ -73,6 +75,44 @@ constexpr int STAGE = 2 * REGION;
 constexpr int FILLS = STAGE / 1024 / 4;    // fill instructions per wave per stage
 __device__ inline int kc_off(int r, int c) { return r * 64 + ((c ^ ((r >> 2) & 3)) << 4); }
 __device__ inline int mc_off(int k, int c) { return k * 512 + ((c ^ ((k & 3) << 2)) << 4); }
+constexpr i64 kGroup = 8;
+// Columns of row tile tm among the columns first .. first + gsz - 1 that are not skipped: from
+// `from` on.  (The caller mirrors C's symmetric top block; BM == BN: a tile below the diagonal holds
+// only elements below it.)
+__host__ __device__ inline i64 row_tiles(i64 upper_rows, i64 tm, i64 first, i64 gsz, i64 &from) {
+  from = (tm + 1) * BM <= upper_rows && tm > first ? tm : first;
+  return first + gsz > from ? first + gsz - from : 0;
+}
+// Tiles of the raster: groups of kGroup column tiles (op(B) side), within a group row by row.
+__host__ __device__ inline i64 group_tiles(i64 upper_rows, i64 tiles_m, i64 first, i64 gsz) {
+  if (upper_rows < BM) return tiles_m * gsz;
+  i64 c = 0, from;
+  for (i64 tm = 0; tm < tiles_m; ++tm) c += row_tiles(upper_rows, tm, first, gsz, from);
+  return c;
+}
+// Tile number idx of the raster.
+__host__ __device__ inline void raster(i64 upper_rows, i64 tiles_m, i64 tiles_n, i64 idx, i64 &tm,
+                                       i64 &tn) {
+  i64 first = 0, gsz;
+  for (;; first += kGroup) {
+    gsz = tiles_n - first < kGroup ? tiles_n - first : kGroup;
+    const i64 c = group_tiles(upper_rows, tiles_m, first, gsz);
+    if (idx < c) break;
+    idx -= c;
+  }
+  if (upper_rows < BM) {
+    tm = idx / gsz;
+    tn = first + idx % gsz;
+    return;
+  }
+  i64 from;
+  for (tm = 0;; ++tm) {
+    const i64 c = row_tiles(upper_rows, tm, first, gsz, from);
+    if (idx < c) break;
+    idx -= c;
+  }
+  tn = from + idx;
+}
 }  // namespace bg
 
 template <bool KA, bool KB>
@@ -86,7 +126,7 @@ __global__ __launch_bounds__(bg::NT) void bf16_gemm_kernel(BgArgs g) {
     else return st2;
   };
   const i64 tiles_m = (g.M + BM - 1) / BM, tiles_n = (g.N + BN - 1) / BN;
-  const i64 total = tiles_m * tiles_n;
+  const i64 total = g.ntiles;
   i64 pid = blockIdx.x;
   if (pid >= total) return;
   {
@@ -96,15 +136,9 @@ __global__ __launch_bounds__(bg::NT) void bf16_gemm_kernel(BgArgs g) {
     const i64 per = total / kXcd, rem = total % kXcd;
     pid = (xcd < rem) ? xcd * (per + 1) + local : rem * (per + 1) + (xcd - rem) * per + local;
   }
-  // grouped raster: groups of kGroup column tiles (op(B) side), the column index fastest
-  constexpr i64 kGroup = 8;
-  const i64 grp = pid / (kGroup * tiles_m), first_n = grp * kGroup;
-  const i64 gsz = (tiles_n - first_n) < kGroup ? (tiles_n - first_n) : kGroup;
-  const i64 within = pid % (kGroup * tiles_m);
-  const i64 m0 = (within / gsz) * BM, n0 = (first_n + within % gsz) * BN;
-  // the caller mirrors C's symmetric top block (BM == BN: a tile below the diagonal holds only
-  // elements below it)
-  if (m0 > n0 && m0 + BM <= g.upper_rows) return;
+  i64 tm, tn;
+  raster(g.upper_rows, tiles_m, tiles_n, g.tile0 + pid, tm, tn);
+  const i64 m0 = tm * BM, n0 = tn * BN;
   const int ks = blockIdx.y;
   const i64 kbeg = (i64)ks * g.kchunk;
   const i64 kend = (kbeg + g.kchunk < g.K) ? kbeg + g.kchunk : g.K;
@@ -267,20 +301,24 @@ __global__ __launch_bounds__(bg::NT) void bf16_gemm_kernel(BgArgs g) {
   }
 
   // epilogue: accumulator registers 4 q0 .. 4 q0 + 3 are four consecutive rows of one column
-  const bool split = g.ksplit > 1;
+  const bool split = g.ksplit > 1 || g.tail;
   float *Cb = split ? g.W + (i64)ks * g.M * g.N : g.C;
-  const i64 ldc = split ? g.M : g.ldc;
+  i64 ldc = split ? g.M : g.ldc, ms = m0, ns = n0, M = g.M, N = g.N;
+  if (g.tail) {  // a whole tile by itself
+    Cb = g.W + (pid * g.ksplit + ks) * (BM * BN);
+    ldc = M = BM, N = BN, ms = ns = 0;
+  }
   const bool vec = (ldc % 4) == 0 && ((reinterpret_cast<uintptr_t>(Cb) & 15) == 0);
 #pragma unroll
   for (int a = 0; a < 4; ++a) {
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
-      const i64 col = n0 + 128 * wc + 32 * b + (lane & 31);
-      if (col >= g.N) continue;
+      const i64 col = ns + 128 * wc + 32 * b + (lane & 31);
+      if (col >= N) continue;
 #pragma unroll
       for (int q0 = 0; q0 < 4; ++q0) {
-        const i64 r = m0 + 128 * wr + 32 * a + 8 * q0 + 4 * (lane >> 5);
-        if (r >= g.M) continue;
+        const i64 r = ms + 128 * wr + 32 * a + 8 * q0 + 4 * (lane >> 5);
+        if (r >= M) continue;
         float *dst = Cb + r + col * ldc;
         f32x4 v = {acc[a][b][4 * q0], acc[a][b][4 * q0 + 1], acc[a][b][4 * q0 + 2],
                    acc[a][b][4 * q0 + 3]};
@@ -288,13 +326,13 @@ __global__ __launch_bounds__(bg::NT) void bf16_gemm_kernel(BgArgs g) {
           v = v * g.alpha;
           if (g.beta != 0.f) {
             for (int q = 0; q < 4; ++q)
-              if (r + q < g.M) v[q] += g.beta * dst[q];
+              if (r + q < M) v[q] += g.beta * dst[q];
           }
         }
-        if (vec && r + 3 < g.M) {
+        if (vec && r + 3 < M) {
           *reinterpret_cast<f32x4 *>(dst) = v;
         } else {
-          for (int q = 0; q < 4 && r + q < g.M; ++q) dst[q] = v[q];
+          for (int q = 0; q < 4 && r + q < M; ++q) dst[q] = v[q];
         }
       }
     }
@@ -314,6 +352,27 @@ __global__ void bf16_splitk_reduce_kernel(i64 M, i64 N, int ksplit, const float 
     float v = alpha * s;
     if (beta != 0.f) v += beta * C[r + c * ldc];
     C[r + c * ldc] = v;
+  }
+}
+
+// C's tile tile0 + blockIdx.x := alpha * the sum of its chunks + beta C (fixed order), 4 columns per
+// blockIdx.y
+__global__ __launch_bounds__(256) void bf16_tail_reduce_kernel(BgArgs g) {
+  using namespace bg;
+  i64 tm, tn;
+  raster(g.upper_rows, (g.M + BM - 1) / BM, (g.N + BN - 1) / BN, g.tile0 + blockIdx.x, tm, tn);
+  const i64 r = tm * BM + 4 * (threadIdx.x & 63), ct = 4 * blockIdx.y + (threadIdx.x >> 6);
+  const i64 c = tn * BN + ct;
+  if (r >= g.M || c >= g.N) return;
+  const float *w = g.W + (i64)blockIdx.x * g.ksplit * (BM * BN) + 4 * (threadIdx.x & 63) + ct * BM;
+  f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int q = 0; q < g.ksplit; ++q) s += *reinterpret_cast<const f32x4 *>(w + (i64)q * (BM * BN));
+  float *dst = g.C + r + c * g.ldc;
+  for (int e = 0; e < 4 && r + e < g.M; ++e) {
+    float v = g.alpha * s[e];
+    if (g.beta != 0.f) v += g.beta * dst[e];
+    dst[e] = v;
   }
 }
 
@@ -356,6 +415,21 @@ struct Operand {
 }  // namespace
 
 namespace {
+
+// K chunks for the last `rem` tiles of a product whose other tiles fill whole rounds of the CUs, 1 when
+// cutting them gains nothing: the rounds they then take at the rate of full ones (1.25 PFLOP/s), and
+// their partial sums' way to memory and back.
+int tail_split(i64 rem, i64 k, i64 rounds) {
+  const double round = 2.0 * bg::BM * bg::BN * (double)k * 256 / 1.25e15;
+  const double part = 2.0 * sizeof(float) * bg::BM * bg::BN * (double)rem / 4e12;
+  int best = 1;
+  double tb = round;
+  for (int s = 2; s <= 16 && k / s >= 16 * bg::BK; ++s) {
+    const double t = round * (double)((rem * s + 255) / 256) / s + part * s + 5e-6;
+    if (t < tb) tb = t, best = s;
+  }
+  return round - tb > 0.04 * round * (double)rounds ? best : 1;
+}
 
 // Shared set-up of gemm_bf16 and gemm_bf16_partials: checks, operand copies where the kernel's
 // alignment rules need them, the split-K choice (at most max_split chunks) and the launch.
@@ -415,12 +489,49 @@ int run_bf16(char ta, char tb, i64 m, i64 n, i64 k, float alpha, const uint16_t 
   } else if (ksplit > 1) {
     g.W = static_cast<float *>(splitk_workspace(sizeof(float) * (size_t)(ksplit * m * n)));
   }
-  dim3 grid((unsigned)tiles, (unsigned)ksplit);
-  if (KA && KB) hipLaunchKernelGGL((bf16_gemm_kernel<true, true>), grid, dim3(bg::NT), 0, ctx().stream, g);
-  else if (KA) hipLaunchKernelGGL((bf16_gemm_kernel<true, false>), grid, dim3(bg::NT), 0, ctx().stream, g);
-  else if (KB) hipLaunchKernelGGL((bf16_gemm_kernel<false, true>), grid, dim3(bg::NT), 0, ctx().stream, g);
-  else hipLaunchKernelGGL((bf16_gemm_kernel<false, false>), grid, dim3(bg::NT), 0, ctx().stream, g);
-  LAUNCH_CHECK();
+  // the tiles that are computed
+  const i64 tiles_m = (m + bg::BM - 1) / bg::BM, tiles_n = (n + bg::BN - 1) / bg::BN;
+  i64 useful = 0;
+  for (i64 first = 0; first < tiles_n; first += bg::kGroup)
+    useful += bg::group_tiles(upper_rows, tiles_m, first,
+                              tiles_n - first < bg::kGroup ? tiles_n - first : bg::kGroup);
+  g.ntiles = useful;
+  auto go = [&](i64 chunks) {
+    const dim3 grid((unsigned)g.ntiles, (unsigned)chunks);
+    if (KA && KB)
+      hipLaunchKernelGGL((bf16_gemm_kernel<true, true>), grid, dim3(bg::NT), 0, ctx().stream, g);
+    else if (KA)
+      hipLaunchKernelGGL((bf16_gemm_kernel<true, false>), grid, dim3(bg::NT), 0, ctx().stream, g);
+    else if (KB)
+      hipLaunchKernelGGL((bf16_gemm_kernel<false, true>), grid, dim3(bg::NT), 0, ctx().stream, g);
+    else
+      hipLaunchKernelGGL((bf16_gemm_kernel<false, false>), grid, dim3(bg::NT), 0, ctx().stream, g);
+    LAUNCH_CHECK();
+  };
+  // A last round that leaves most CUs idle is cut in K: 8192 x 4096 x 131072 with its symmetric half
+  // skipped is 392 tiles, one and a half rounds that took two: 6.87 -> 6.02 ms (3.70 + 2.20 + 0.13).
+  if (!W && ksplit == 1 && ctx().max_wgs == 0 && useful > kCUs && useful <= 8 * kCUs &&
+      useful % kCUs != 0) {
+    const i64 rem = useful % kCUs;
+    const int s = tail_split(rem, k, (useful + kCUs - 1) / kCUs);
+    const size_t bytes = sizeof(float) * (size_t)(rem * s) * bg::BM * bg::BN;
+    if (s > 1 && bytes <= splitk_budget()) {
+      g.ntiles = useful - rem;
+      go(1);
+      g.W = static_cast<float *>(splitk_workspace(bytes));
+      g.tile0 = useful - rem;
+      g.ntiles = rem;
+      g.tail = 1;
+      g.kchunk = ((k + s - 1) / s + bg::BK - 1) / bg::BK * bg::BK;
+      g.ksplit = (int)((k + g.kchunk - 1) / g.kchunk);
+      go(g.ksplit);
+      hipLaunchKernelGGL(bf16_tail_reduce_kernel, dim3((unsigned)rem, bg::BN / 4), dim3(256), 0,
+                         ctx().stream, g);
+      LAUNCH_CHECK();
+      return 1;
+    }
+  }
+  go(ksplit);
   if (!W && ksplit > 1) {
     i64 blocks = (m * n + 255) / 256;
     if (blocks > 4096) blocks = 4096;
