@@ -543,7 +543,7 @@ def main():
     # timed with HIP events on the library's stream, exactly one launch when Omega is supplied
     flop = 2.0 * m * n * Nl
     t_sketch = stage_avg[0]
-    kname = "isvd::gemm_dl_kernel<false,false>" if oa == "C" else "isvd::gemm_dl_kernel<false,true>"
+    kname = f"isvd::gemm_stream_kernel<double,{'false' if oa == 'C' else 'true'},4,2>"
     roofline = {"bound": "mfma", "achieved": flop / t_sketch / 1e12,
                 "peak": PEAK_FP64_MFMA / 1e12, "unit": "TFLOP/s",
                 "frac": flop / t_sketch / PEAK_FP64_MFMA, "traffic": traffic_of(kname),
