@@ -859,8 +859,9 @@ StreamPlan stream_plan(const GemmArgs<T> &g, bool KB, i64 batch) {
   using X = stream::Traits<T>;
   StreamPlan p;
   if (g.ct || g.tiled || batch > 1024) return p;
-  // per-lane offsets are 32-bit byte counts below 16 * 8 leading dimensions
-  if (g.lda >= (1 << 22) || g.ldb >= (1 << 22)) return p;
+  // per-lane offsets are 32-bit byte counts: 64 doubles or 128 floats apart in a K-contiguous B's
+  // columns, 3 V rows of A and 3 rows of an N-contiguous B
+  if (g.lda >= (1 << 25) || g.ldb >= (KB ? 1 << 23 : 1 << 26)) return p;
   const i64 min_chunk = 16 * X::STEP;
   if (g.m <= 64) {
     // Few rows against a large op(B), from K = 1024 and n = 256 on (below, a product is a few
@@ -925,7 +926,7 @@ void launch_stream(GemmArgs<T> g, const StreamPlan &p, i64 batch) {
   if (ctx().max_wgs > 0)
     while (ks > 1 && p.blocks * batch * ks > ctx().max_wgs) --ks;
   const size_t per = sizeof(T) * (size_t)(batch * g.m * g.n);
-  while (ks > 1 && per * (size_t)ks > splitk_budget()) --ks;
+  while (ks > 1 && (per * (size_t)ks > splitk_budget() || batch * ks > 65535)) --ks;
   i64 kchunk = (g.k + ks - 1) / ks;
   kchunk = (kchunk + X::STEP - 1) / X::STEP * X::STEP;
   ks = (g.k + kchunk - 1) / kchunk;
