@@ -13,11 +13,12 @@
 // A PSD matrix is factored by Cholesky in place first, W = L L^T, and the iteration runs on L,
 // whose singular values are the roots of W's: 9-10 sweeps instead of 13-15.
 //
-// Measured, FP64 (one rotation a round with the vectors of V in global memory before): V and U at
-// l = 64 660 -> 346 + 47 us, l = 128 3570 -> 1570 + 106 us; PSD at l = 48 450 -> 190 us, l = 128
-// 3000 -> 1250 us.  Bound by instruction issue: the vector unit is busy 50 % (l = 64, one wave per
-// SIMD) to 60 % (l = 128, two) of the time, the rest waits for LDS, barriers and dependent FP64
-// results; four groups of lanes per pair instead of two, or eight lanes a group, were slower.
+// Measured, FP64, 256 x 256 matrices with singular values down to 4 % (one rotation a round, with the
+// vectors of V in global memory and every norm summed at every rotation, before): V and U at l = 64
+// 618 -> 386 + 53 us, l = 128 4050 -> 1677 + 118 us; PSD at l = 48 485 -> 280 us, l = 128 3084 -> 1777
+// us.  Bound by instruction issue: the vector unit is busy 50 % (l = 64, one wave per SIMD) to 60 %
+// (l = 128, two) of the time, the rest waits for LDS, barriers and dependent FP64 results; four groups
+// of lanes per pair instead of two, or eight lanes a group, were slower.
 #include "la.hpp"
 
 #include <type_traits>
@@ -31,19 +32,27 @@ namespace isvd {
 namespace {
 
 template <typename T> struct Eps;
-template <> struct Eps<double> { static constexpr double v = DBL_EPSILON; };
-template <> struct Eps<float> { static constexpr float v = FLT_EPSILON; };
+template <> struct Eps<double> {
+  static constexpr double v = DBL_EPSILON, least = DBL_MIN;
+  static constexpr int exponent = 0;  // see the load
+};
+template <> struct Eps<float> {
+  static constexpr float v = FLT_EPSILON, least = FLT_MIN;
+  static constexpr int exponent = 22;
+};
 
 constexpr int kMaxSweeps = 40;
 // 16 lanes per block pair, each holding every 16th row of its four columns
 constexpr int kTpp = 16;
 constexpr int kMaxThreads = 512;  // n = 128: 32 groups
 
-// the hardware's approximations (FP64: about 1e-8 relative; FP32: 1 ulp)
-__device__ __forceinline__ double rcp_approx(double x) { return __builtin_amdgcn_rcp(x); }
-__device__ __forceinline__ double rsq_approx(double x) { return __builtin_amdgcn_rsq(x); }
-__device__ __forceinline__ float rcp_approx(float x) { return __builtin_amdgcn_rcpf(x); }
-__device__ __forceinline__ float rsq_approx(float x) { return __builtin_amdgcn_rsqf(x); }
+// x^(-1/2): FP64 the hardware's approximation (better than 2^-23) through one step of third order, FP32
+// the hardware's (1 ulp)
+__device__ __forceinline__ double rsq(double x) {
+  const double r = __builtin_amdgcn_rsq(x), e = 1.0 - (x * r) * r;
+  return r + (r * e) * (0.375 * e + 0.5);
+}
+__device__ __forceinline__ float rsq(float x) { return __builtin_amdgcn_rsqf(x); }
 
 // rows per lane for an n x n problem (a power of two)
 inline int jacobi_rpl(i64 n) {
@@ -71,9 +80,23 @@ __device__ __forceinline__ void rr_pair(int np, int r, int k, int &p, int &q) {
 // 0, for group k, the two rotations inside the blocks it starts with, (p0, p1), (q0, q1); in slot
 // 1 + r, r < 2 g - 1, the four cross rotations of its block pair in outer round r, (p0, q0),
 // (p1, q1), (p0, q1), (p1, q0).
+// A rotation: cos and sin in FP64.  In FP32 t = tan(theta / 2) stands for the cosine, c = 1 - s t: next
+// to 1 it has the digits that a cosine rounds away, a few hundred rotations of which had moved the
+// singular values by up to n units of roundoff.
 template <typename T>
 struct Rot {
   T c, s;
+  static __device__ Rot none() { return {T(sizeof(T) == 8 ? 1 : 0), T(0)}; }
+  __device__ __forceinline__ void turn(T &a, T &b) const {
+    const T x = a, y = b;
+    if constexpr (sizeof(T) == 8) {
+      a = c * x - s * y;
+      b = s * x + c * y;
+    } else {
+      a = x - s * (c * x + y);
+      b = y + s * (x - c * y);
+    }
+  }
 };
 __host__ __device__ inline i64 log_entries(int groups) {
   return (i64)kMaxSweeps * 2 * groups * groups * 4;
@@ -101,6 +124,7 @@ __global__ __launch_bounds__(kMaxThreads) void svd_jacobi_kernel(
   __shared__ int rank_of[128];
   __shared__ int n_rot;
   __shared__ T shift_sh;
+  __shared__ int exp_sh;
 
   const int b = blockIdx.x;
   const int tid = threadIdx.x;
@@ -113,17 +137,40 @@ __global__ __launch_bounds__(kMaxThreads) void svd_jacobi_kernel(
   constexpr int ld = R + 1;
 
   // ---- load (rows n .. R-1 and columns n .. zero) ----
-  auto load = [&](bool upper) {
+  auto load = [&](bool upper, int sh) {
     for (int e = tid; e < R * cols; e += nt) {
       const int i = e % R, j = e / R;
       T v = T(0);
       if (i < n && j < n)
         v = (upper && i > j) ? Ab[j + (i64)i * lda] : Ab[i + (i64)j * lda];
-      G[i + j * ld] = v;
+      G[i + j * ld] = ldexp(v, -sh);
     }
     __syncthreads();
   };
-  load(mode != kGeneral);
+  load(mode != kGeneral, 0);
+  // The largest entry to 2^(exponent - 1) .. 2^exponent, by a power of two (exactly): the squares of
+  // squared norms stay below overflow, and above underflow for columns down to 1e-77 (FP32: 1e-16)
+  // of the largest.  Everything below is on the scaled matrix up to what is stored.
+  {
+    T top = 0;
+    for (int e = tid; e < R * cols; e += nt) top = fmax(top, fabs(G[e % R + (e / R) * ld]));
+    for (int off = 32; off; off >>= 1) top = fmax(top, __shfl_xor(top, off, 64));
+    if ((tid & 63) == 0) red[tid >> 6] = top;
+    __syncthreads();
+    if (tid == 0) {
+      for (int w = 1; w < waves; ++w) top = fmax(top, red[w]);
+      int ex = Eps<T>::exponent;
+      if (top > T(0) && top < T(INFINITY)) (void)frexp(top, &ex);
+      exp_sh = ex - Eps<T>::exponent;
+    }
+    __syncthreads();
+  }
+  const int sh = exp_sh;
+  for (int e = tid; e < R * cols; e += nt) {
+    T &g = G[e % R + (e / R) * ld];
+    g = ldexp(g, -sh);
+  }
+  __syncthreads();
   if (mode == kSymmetric) {
     // c = 2 ||A||_F (+1 when A == 0), deterministic block reduction
     T part = 0;
@@ -176,22 +223,27 @@ __global__ __launch_bounds__(kMaxThreads) void svd_jacobi_kernel(
       __syncthreads();
     } else {
       __syncthreads();
-      load(true);
+      load(true, sh);
     }
   }
 
-  // FP32 keeps rotating to 4 units of roundoff (the dot products are good to about one), or the
-  // directions would be off by n of them over the gap of their singular values
-  const T tol = sizeof(T) == 8 ? Eps<T>::v * T(n) : T(4) * Eps<T>::v;
+  // Rotations down to 4 units of roundoff (the dot products are good to about one), or the directions
+  // would be off by n of them over the gap of their singular values (n units of them: half a sweep
+  // less on average, vectors of a PSD matrix of 64 columns 4 times as far off)
+  const T tol = T(4) * Eps<T>::v;
   const T tol2 = tol * tol;
   // Two rotations side by side, columns (a0, b0) and (a1, b1) with squared norms na, nb.  With
-  // zeta = (nb - na) / (2 gamma) = cot(2 theta): r = (1 + zeta^2)^(-1/2), c^2 = (1 + |zeta| r) / 2,
-  // s = sign(zeta) r / (2 c), from the reciprocal (square root) instructions as they are, to about
-  // 1e-8: an angle off by that leaves 1e-8 gamma behind, which the next sweep takes.  What has to
-  // be exact is c^2 + s^2 = 1: both are scaled by (1 + e)^(-1/2), e = c^2 + s^2 - 1, to third order.
-  // (Exact divisions and roots: 110 ns more a round.)
+  // d = nb - na and h = 2 gamma, d : h = cot(2 theta): r = (d^2 + h^2)^(-1/2), c^2 = (1 + |d| r) / 2,
+  // s = sign(d) h r / (2 c).  A pair with d^2 + h^2 below the smallest normal number is not rotated
+  // (both columns are as good as zero).  (With divisions and the library's roots: 110 ns more a round.)
   typedef T Col[RPL];
   int rotated = 0;
+  auto sum_sq = [&](const Col &x) {
+    T v = 0;
+#pragma unroll
+    for (int u = 0; u < RPL; ++u) v += x[u] * x[u];
+    return lane_group_sum(v, kTpp);
+  };
   auto rot2 = [&](Col &a0, Col &b0, T &na0, T &nb0, Col &a1, Col &b1, T &na1, T &nb1,
                   Rot<T> *out) {
     T g0 = 0, g1 = 0;
@@ -202,35 +254,30 @@ __global__ __launch_bounds__(kMaxThreads) void svd_jacobi_kernel(
     }
     g0 = lane_group_sum(g0, kTpp);
     g1 = lane_group_sum(g1, kTpp);
+    const T d0 = nb0 - na0, h0 = T(2) * g0, q0 = d0 * d0 + h0 * h0;
+    const T d1 = nb1 - na1, h1 = T(2) * g1, q1 = d1 * d1 + h1 * h1;
     // |gamma| > tol sqrt(alpha beta), compared in squares
-    const bool n0 = g0 * g0 > tol2 * (na0 * nb0), n1 = g1 * g1 > tol2 * (na1 * nb1);
-    Rot<T> r0{T(1), T(0)}, r1{T(1), T(0)};
+    const bool n0 = g0 * g0 > tol2 * (na0 * nb0) && q0 >= Eps<T>::least;
+    const bool n1 = g1 * g1 > tol2 * (na1 * nb1) && q1 >= Eps<T>::least;
+    Rot<T> r0 = Rot<T>::none(), r1 = r0;
     if (n0 || n1) {
-      auto angle = [&](bool need, T g, T &na, T &nb) {
-        const T zeta = (nb - na) * rcp_approx(T(2) * g);
-        const T r = rsq_approx(T(1) + zeta * zeta);
-        const T c2 = T(0.5) + T(0.5) * fabs(zeta) * r;
-        const T y = rsq_approx(c2);
-        T c = c2 * y, s = T(0.5) * r * y;
-        const T e = c * c + (s * s - T(1));
-        const T f = T(1) + e * (T(0.375) * e - T(0.5));
-        c = need ? c * f : T(1);
-        s = need ? (zeta >= T(0) ? s * f : -(s * f)) : T(0);
-        const T g2 = T(2) * c * s * g, cc = c * c, ss = s * s;
+      auto angle = [&](bool need, T d, T h, T q, T &na, T &nb) {
+        const T r = rsq(q), c2 = T(0.5) + T(0.5) * fabs(d) * r, z = rsq(c2);
+        const T c = need ? c2 * z : T(1), sa = T(0.5) * h * r * z;
+        const T s = need ? (d >= T(0) ? sa : -sa) : T(0);
+        const T g2 = c * s * h, cc = c * c, ss = s * s;
         const T xa = (cc * na - g2) + ss * nb, xb = (ss * na + g2) + cc * nb;
-        na = xa;
-        nb = xb;
-        return Rot<T>{c, s};
+        na = fmax(xa, T(0));
+        nb = fmax(xb, T(0));
+        if constexpr (sizeof(T) == 8) return Rot<T>{c, s};
+        else return Rot<T>{s * __builtin_amdgcn_rcpf(T(1) + c), s};
       };
-      r0 = angle(n0, g0, na0, nb0);
-      r1 = angle(n1, g1, na1, nb1);
+      r0 = angle(n0, d0, h0, q0, na0, nb0);
+      r1 = angle(n1, d1, h1, q1, na1, nb1);
 #pragma unroll
       for (int u = 0; u < RPL; ++u) {
-        const T x0 = a0[u], y0 = b0[u], x1 = a1[u], y1 = b1[u];
-        a0[u] = r0.c * x0 - r0.s * y0;
-        b0[u] = r0.s * x0 + r0.c * y0;
-        a1[u] = r1.c * x1 - r1.s * y1;
-        b1[u] = r1.s * x1 + r1.c * y1;
+        r0.turn(a0[u], b0[u]);
+        r1.turn(a1[u], b1[u]);
       }
       rotated = 1;
     }
@@ -262,19 +309,12 @@ __global__ __launch_bounds__(kMaxThreads) void svd_jacobi_kernel(
         if (r == 0) {
           // squared norms afresh; within the sweep each rotation updates its two (a sweep without a
           // rotation, which ends the iteration, thus tested every pair against norms of its
-          // columns); the rotations inside the blocks
-          np0 = np1 = nq0 = nq1 = T(0);
-#pragma unroll
-          for (int u = 0; u < RPL; ++u) {
-            np0 += p0[u] * p0[u];
-            np1 += p1[u] * p1[u];
-            nq0 += q0[u] * q0[u];
-            nq1 += q1[u] * q1[u];
-          }
-          np0 = lane_group_sum(np0, kTpp);
-          np1 = lane_group_sum(np1, kTpp);
-          nq0 = lane_group_sum(nq0, kTpp);
-          nq1 = lane_group_sum(nq1, kTpp);
+          // columns; the norm of a column that collapses onto another is rounding until then, and
+          // a rotation with it no more than a needless one); the rotations inside the blocks
+          np0 = sum_sq(p0);
+          np1 = sum_sq(p1);
+          nq0 = sum_sq(q0);
+          nq1 = sum_sq(q1);
           rot2(p0, p1, np0, np1, q0, q1, nq0, nq1, lg + (i64)sweep * blocks * 4 * groups + grp);
         } else {
           np0 = nrm[2 * P];
@@ -325,8 +365,8 @@ __global__ __launch_bounds__(kMaxThreads) void svd_jacobi_kernel(
   }
   __syncthreads();
   for (int j = tid; j < n; j += nt)
-    sig[(i64)b * lds + rank_of[j]] = factored ? nrm[j] * nrm[j] : nrm[j];
-  if (mode == kSymmetric && tid == 0 && shift_out) shift_out[b] = shift_sh;
+    sig[(i64)b * lds + rank_of[j]] = ldexp(factored ? nrm[j] * nrm[j] : nrm[j], sh);
+  if (mode == kSymmetric && tid == 0 && shift_out) shift_out[b] = ldexp(shift_sh, sh);
   if (U) {
     T *Ub = U + (i64)b * sU;
     for (int e = tid; e < n * n; e += nt) {
@@ -346,7 +386,7 @@ __global__ __launch_bounds__(kMaxThreads) void svd_jacobi_kernel(
 // lives in the registers of `seg` lanes (a power of two >= groups), lane k holding the entries of
 // the block pair at table k, and between outer rounds the blocks move to the next table as the
 // players of the circle do: p to the left, q to the right, turning at both ends.  No barrier, no
-// LDS; the log is read eight outer rounds ahead.  128 x 128 FP64, 10 sweeps: 106 us (64 x 64: 47 us).
+// LDS; the log is read eight outer rounds ahead.  128 x 128 FP64, 11 sweeps: 118 us (64 x 64: 53 us).
 template <typename T>
 __device__ __forceinline__ T from_next(T v) { return dpp_mov<0x130>(v); }  // lane i: lane i + 1's
 template <typename T>
@@ -368,11 +408,6 @@ __global__ __launch_bounds__(256) void jacobi_replay_kernel(int n, int seg,
   // the entries of this lane's blocks in round 0: P = k, Q = last block (k = 0) or blocks - 1 - k
   const int P = kc, Q = kc == 0 ? blocks - 1 : blocks - 1 - kc;
   T p0 = row == 2 * P, p1 = row == 2 * P + 1, q0 = row == 2 * Q, q1 = row == 2 * Q + 1;
-  auto rot = [](const Rot<T> &r, T &a, T &c) {
-    const T x = a, y = c;
-    a = r.c * x - r.s * y;
-    c = r.s * x + r.c * y;
-  };
   constexpr int AHEAD = 8;
   struct Slot {
     Rot<T> r[4];
@@ -397,13 +432,13 @@ __global__ __launch_bounds__(256) void jacobi_replay_kernel(int n, int seg,
         buf[a] = fetch(i0 + a + AHEAD);
         if (i0 + a < total) {
           if (slot == 0) {
-            rot(s.r[0], p0, p1);
-            rot(s.r[1], q0, q1);
+            s.r[0].turn(p0, p1);
+            s.r[1].turn(q0, q1);
           } else {
-            rot(s.r[0], p0, q0);
-            rot(s.r[1], p1, q1);
-            rot(s.r[2], p0, q1);
-            rot(s.r[3], p1, q0);
+            s.r[0].turn(p0, q0);
+            s.r[1].turn(p1, q1);
+            s.r[2].turn(p0, q1);
+            s.r[3].turn(p1, q0);
             if (groups > 1) {
               // p_k := p_{k+1}, p_last := q_last; q_k := q_{k-1} (k >= 2), q_1 := p_0; q_0 stays
               const T np0 = from_next(p0), np1 = from_next(p1);
