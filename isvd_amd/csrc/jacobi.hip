@@ -21,6 +21,7 @@
 // of lanes per pair instead of two, or eight lanes a group, were slower.
 #include "la.hpp"
 
+#include <algorithm>
 #include <type_traits>
 
 #include "dpp.hpp"
@@ -42,6 +43,12 @@ template <> struct Eps<float> {
 };
 
 constexpr int kMaxSweeps = 40;
+// Sweeps the rotation log holds.  Ten or eleven are the rule; columns that collapse onto each other can
+// take more, and the rotations so far are then replayed on V before the log starts over.
+constexpr int kLogSweeps = 16;
+// Bytes the logs of one launch may take: a round of the CUs at n = 128 (256 problems of 2.1 MB in
+// FP64), several below.  Larger batches go in several launches.
+constexpr size_t kLogBytes = 640ull << 20;
 // 16 lanes per block pair, each holding every 16th row of its four columns
 constexpr int kTpp = 16;
 constexpr int kMaxThreads = 512;  // n = 128: 32 groups
@@ -99,10 +106,100 @@ struct Rot {
   }
 };
 __host__ __device__ inline i64 log_entries(int groups) {
-  return (i64)kMaxSweeps * 2 * groups * groups * 4;
+  return (i64)kLogSweeps * 2 * groups * groups * 4;
+}
+
+// One row of V through `slots` slots of the rotation log lg: row i of V is e_i^T (resume: row i of V as
+// it is) through the rotations in order.  A row lives in the registers of consecutive lanes (groups of
+// them, padded to a power of two), lane k holding the entries of the block pair at table k, and
+// between outer rounds the blocks move to the next table as the players of the circle do: p to the
+// left, q to the right, turning at both ends.  No barrier, no LDS; the log is read AHEAD outer rounds
+// ahead.  Column j of the row is stored as column rank[j] (rank null: j).
+template <typename T>
+__device__ __forceinline__ T from_next(T v) { return dpp_mov<0x130>(v); }  // lane i: lane i + 1's
+template <typename T>
+__device__ __forceinline__ T from_prev(T v) { return dpp_mov<0x138>(v); }  // lane i: lane i - 1's
+
+template <typename T, int AHEAD>
+__device__ __forceinline__ void replay_row(int n, int k, int row, const Rot<T> *lg, int slots,
+                                           bool resume, const int *rank, T *V, i64 ldv) {
+  const int groups = jacobi_groups(n), blocks = 2 * groups;
+  const bool live = k < groups;
+  const int kc = live ? k : 0;
+  // the entries of this lane's blocks in round 0: P = k, Q = last block (k = 0) or blocks - 1 - k
+  const int P = kc, Q = kc == 0 ? blocks - 1 : blocks - 1 - kc;
+  auto entry = [&](int col) -> T {
+    if (!resume) return T(row == col);
+    return row < n && col < n ? V[row + (i64)col * ldv] : T(0);
+  };
+  T p0 = entry(2 * P), p1 = entry(2 * P + 1), q0 = entry(2 * Q), q1 = entry(2 * Q + 1);
+  struct Slot {
+    Rot<T> r[4];
+  };
+  auto fetch = [&](int i) {
+    const int c = i < slots ? i : slots - 1;
+    Slot v;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v.r[j] = lg[((i64)c * 4 + j) * groups + kc];
+    return v;
+  };
+  if (slots > 0) {
+    Slot buf[AHEAD];
+#pragma unroll
+    for (int a = 0; a < AHEAD; ++a) buf[a] = fetch(a);
+    int slot = 0;  // of the sweep
+    for (int i0 = 0; i0 < slots; i0 += AHEAD) {
+#pragma unroll
+      for (int a = 0; a < AHEAD; ++a) {
+        const Slot s = buf[a];
+        buf[a] = fetch(i0 + a + AHEAD);
+        if (i0 + a < slots) {
+          if (slot == 0) {
+            s.r[0].turn(p0, p1);
+            s.r[1].turn(q0, q1);
+          } else {
+            s.r[0].turn(p0, q0);
+            s.r[1].turn(p1, q1);
+            s.r[2].turn(p0, q1);
+            s.r[3].turn(p1, q0);
+            if (groups > 1) {
+              // p_k := p_{k+1}, p_last := q_last; q_k := q_{k-1} (k >= 2), q_1 := p_0; q_0 stays
+              const T np0 = from_next(p0), np1 = from_next(p1);
+              const T nq0 = from_prev(k == 0 ? p0 : q0), nq1 = from_prev(k == 0 ? p1 : q1);
+              const bool last = k == groups - 1;
+              const T lp0 = last ? q0 : np0, lp1 = last ? q1 : np1;
+              q0 = k == 0 ? q0 : nq0;
+              q1 = k == 0 ? q1 : nq1;
+              p0 = lp0;
+              p1 = lp1;
+            }
+          }
+          slot = slot + 1 == blocks ? 0 : slot + 1;
+        }
+      }
+    }
+  }
+  if (row >= n || !live) return;
+  // whole sweeps leave every block where it started
+  auto store = [&](int col, T v) {
+    if (col < n) V[row + (i64)(rank ? rank[col] : col) * ldv] = v;
+  };
+  store(2 * P, p0);
+  store(2 * P + 1, p1);
+  store(2 * Q, q0);
+  store(2 * Q + 1, q1);
+}
+
+// lanes a row takes
+__host__ __device__ inline int replay_lanes(int groups) {
+  int seg = 1;
+  while (seg < groups) seg *= 2;
+  return seg;
 }
 
 enum { kGeneral = 0, kSymmetric = 1, kPsd = 2 };
+// per problem: the columns' ranks, the sweeps in the log, whether V holds those before it
+constexpr int kOrder = 132, kOrderSweeps = 128, kOrderResume = 129;
 
 // kGeneral: SVD of A (general n x n).  kSymmetric: symmetric eigendecomposition of the matrix whose
 // upper triangle is stored in A, computed as the SVD of sym(A) + c I with c = 2 ||sym(A)||_F.
@@ -114,8 +211,8 @@ enum { kGeneral = 0, kSymmetric = 1, kPsd = 2 };
 template <typename T, int RPL>
 __global__ __launch_bounds__(kMaxThreads) void svd_jacobi_kernel(
     int n, int mode, const T *__restrict__ A, i64 lda, i64 sA, T *__restrict__ sig, i64 lds,
-    T *__restrict__ U, i64 ldu, i64 sU, Rot<T> *__restrict__ log, int *__restrict__ order,
-    T *__restrict__ shift_out) {
+    T *__restrict__ U, i64 ldu, i64 sU, T *V, i64 ldv, i64 sV, Rot<T> *__restrict__ log,
+    int *__restrict__ order, T *__restrict__ shift_out) {
   extern __shared__ unsigned char smem_raw[];
   // leading dimension 16 RPL + 1: the columns a wave works on start in different banks
   T *G = reinterpret_cast<T *>(smem_raw);
@@ -287,14 +384,24 @@ __global__ __launch_bounds__(kMaxThreads) void svd_jacobi_kernel(
     }
   };
   Rot<T> *lg = log ? log + (i64)b * log_entries(groups) : nullptr;
-  int sweep = 0;
-  for (; sweep < kMaxSweeps; ++sweep) {
+  int logged = 0;  // sweeps in the log
+  bool resume = false;
+  for (int sweep = 0; sweep < kMaxSweeps; ++sweep) {
+    if (log && logged == kLogSweeps) {
+      const int lane = tid & 63, seg = replay_lanes(groups), rows = 64 / seg;
+      for (int r0 = (tid >> 6) * rows; r0 < n; r0 += waves * rows)
+        replay_row<T, 2>(n, lane % seg, r0 + lane / seg, lg, logged * blocks, resume, nullptr,
+                         V + (i64)b * sV, ldv);
+      resume = true;
+      logged = 0;
+      __syncthreads();
+    }
     if (tid == 0) n_rot = 0;
     rotated = 0;
     for (int r = 0; r < blocks - 1; ++r) {
       int P = 0, Q = 1;
       if (live) rr_pair(blocks, r, grp, P, Q);
-      Rot<T> *out = lg + ((i64)sweep * blocks + 1 + r) * 4 * groups + grp;
+      Rot<T> *out = lg + ((i64)logged * blocks + 1 + r) * 4 * groups + grp;
       if (live) {
         T *cp = G + 2 * P * ld + sub, *cq = G + 2 * Q * ld + sub;
         Col p0, p1, q0, q1;
@@ -315,7 +422,7 @@ __global__ __launch_bounds__(kMaxThreads) void svd_jacobi_kernel(
           np1 = sum_sq(p1);
           nq0 = sum_sq(q0);
           nq1 = sum_sq(q1);
-          rot2(p0, p1, np0, np1, q0, q1, nq0, nq1, lg + (i64)sweep * blocks * 4 * groups + grp);
+          rot2(p0, p1, np0, np1, q0, q1, nq0, nq1, lg + (i64)logged * blocks * 4 * groups + grp);
         } else {
           np0 = nrm[2 * P];
           np1 = nrm[2 * P + 1];
@@ -344,6 +451,7 @@ __global__ __launch_bounds__(kMaxThreads) void svd_jacobi_kernel(
     const int go = n_rot;
     __syncthreads();
     if (go == 0) break;
+    ++logged;
   }
 
   // ---- singular values (column norms), ranks for descending order ----
@@ -376,94 +484,27 @@ __global__ __launch_bounds__(kMaxThreads) void svd_jacobi_kernel(
     }
   }
   if (order) {
-    // the columns' ranks, then the sweeps that rotated anything
-    for (int j = tid; j < n; j += nt) order[b * 132 + j] = rank_of[j];
-    if (tid == 0) order[b * 132 + 128] = sweep;
+    for (int j = tid; j < n; j += nt) order[b * kOrder + j] = rank_of[j];
+    if (tid == 0) {
+      order[b * kOrder + kOrderSweeps] = logged;
+      order[b * kOrder + kOrderResume] = resume;
+    }
   }
 }
 
-// V of the SVD from the rotation log: row i of V is e_i^T through the rotations in order.  A row
-// lives in the registers of `seg` lanes (a power of two >= groups), lane k holding the entries of
-// the block pair at table k, and between outer rounds the blocks move to the next table as the
-// players of the circle do: p to the left, q to the right, turning at both ends.  No barrier, no
-// LDS; the log is read eight outer rounds ahead.  128 x 128 FP64, 11 sweeps: 118 us (64 x 64: 53 us).
-template <typename T>
-__device__ __forceinline__ T from_next(T v) { return dpp_mov<0x130>(v); }  // lane i: lane i + 1's
-template <typename T>
-__device__ __forceinline__ T from_prev(T v) { return dpp_mov<0x138>(v); }  // lane i: lane i - 1's
-
+// V of the SVD from the rotation log, a row per `seg` lanes, the log read eight outer rounds ahead.
+// 128 x 128 FP64, 11 sweeps: 118 us (64 x 64: 53 us).
 template <typename T>
 __global__ __launch_bounds__(256) void jacobi_replay_kernel(int n, int seg,
                                                             const Rot<T> *__restrict__ log,
-                                                            const int *__restrict__ order,
-                                                            T *__restrict__ V, i64 ldv, i64 sV) {
-  const int groups = jacobi_groups(n), blocks = 2 * groups;
+                                                            const int *__restrict__ order, T *V,
+                                                            i64 ldv, i64 sV) {
+  const int groups = jacobi_groups(n);
   const int b = blockIdx.y, lane = threadIdx.x & 63;
-  const int k = lane % seg;  // table
   const int row = (blockIdx.x * 4 + (threadIdx.x >> 6)) * (64 / seg) + lane / seg;
-  const int sweeps = order[b * 132 + 128];
-  const Rot<T> *lg = log + (i64)b * log_entries(groups);
-  const bool live = k < groups;
-  const int kc = live ? k : 0;
-  // the entries of this lane's blocks in round 0: P = k, Q = last block (k = 0) or blocks - 1 - k
-  const int P = kc, Q = kc == 0 ? blocks - 1 : blocks - 1 - kc;
-  T p0 = row == 2 * P, p1 = row == 2 * P + 1, q0 = row == 2 * Q, q1 = row == 2 * Q + 1;
-  constexpr int AHEAD = 8;
-  struct Slot {
-    Rot<T> r[4];
-  };
-  const int total = sweeps * blocks;
-  auto fetch = [&](int i) {
-    const int c = i < total ? i : total - 1;
-    Slot v;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) v.r[j] = lg[((i64)c * 4 + j) * groups + kc];
-    return v;
-  };
-  if (total > 0) {
-    Slot buf[AHEAD];
-#pragma unroll
-    for (int a = 0; a < AHEAD; ++a) buf[a] = fetch(a);
-    int slot = 0;  // of the sweep
-    for (int i0 = 0; i0 < total; i0 += AHEAD) {
-#pragma unroll
-      for (int a = 0; a < AHEAD; ++a) {
-        const Slot s = buf[a];
-        buf[a] = fetch(i0 + a + AHEAD);
-        if (i0 + a < total) {
-          if (slot == 0) {
-            s.r[0].turn(p0, p1);
-            s.r[1].turn(q0, q1);
-          } else {
-            s.r[0].turn(p0, q0);
-            s.r[1].turn(p1, q1);
-            s.r[2].turn(p0, q1);
-            s.r[3].turn(p1, q0);
-            if (groups > 1) {
-              // p_k := p_{k+1}, p_last := q_last; q_k := q_{k-1} (k >= 2), q_1 := p_0; q_0 stays
-              const T np0 = from_next(p0), np1 = from_next(p1);
-              const T nq0 = from_prev(k == 0 ? p0 : q0), nq1 = from_prev(k == 0 ? p1 : q1);
-              const bool last = k == groups - 1;
-              const T lp0 = last ? q0 : np0, lp1 = last ? q1 : np1;
-              q0 = k == 0 ? q0 : nq0;
-              q1 = k == 0 ? q1 : nq1;
-              p0 = lp0;
-              p1 = lp1;
-            }
-          }
-          slot = slot + 1 == blocks ? 0 : slot + 1;
-        }
-      }
-    }
-  }
-  if (row >= n || !live) return;
-  // whole sweeps leave every block where it started
-  T *Vb = V + (i64)b * sV;
-  const int *rk = order + b * 132;
-  if (2 * P < n) Vb[row + (i64)rk[2 * P] * ldv] = p0;
-  if (2 * P + 1 < n) Vb[row + (i64)rk[2 * P + 1] * ldv] = p1;
-  if (2 * Q < n) Vb[row + (i64)rk[2 * Q] * ldv] = q0;
-  if (2 * Q + 1 < n) Vb[row + (i64)rk[2 * Q + 1] * ldv] = q1;
+  const int *o = order + b * kOrder;
+  replay_row<T, 8>(n, lane % seg, row, log + (i64)b * log_entries(groups),
+                   o[kOrderSweeps] * 2 * groups, o[kOrderResume] != 0, o, V + (i64)b * sV, ldv);
 }
 
 // eigenvalues ascending from the shifted SVD: w[j] = sig[n-1-j] - c, Z[:, j] = U[:, n-1-j]
@@ -480,7 +521,7 @@ __global__ void syev_finish_kernel(int n, const T *sig, const T *shift, const T 
 
 template <typename T, int RPL>
 void launch_rpl(i64 n, int mode, const T *A, i64 lda, i64 sA, T *s, i64 lds, T *U, i64 ldu, i64 sU,
-                i64 batch, Rot<T> *log, int *order, T *shift_out) {
+                T *V, i64 ldv, i64 sV, i64 batch, Rot<T> *log, int *order, T *shift_out) {
   const int groups = jacobi_groups((int)n);
   const size_t shmem = sizeof(T) * (size_t)(kTpp * RPL + 1) * (size_t)(4 * groups);
   const int nt = (groups * kTpp + 63) / 64 * 64;
@@ -488,7 +529,7 @@ void launch_rpl(i64 n, int mode, const T *A, i64 lda, i64 sA, T *s, i64 lds, T *
   HIP_CHECK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)shmem));
   hipLaunchKernelGGL(kern, dim3((unsigned)batch), dim3(nt), shmem, ctx().stream, (int)n, mode, A,
-                     lda, sA, s, lds, U, ldu, sU, log, order, shift_out);
+                     lda, sA, s, lds, U, ldu, sU, V, ldv, sV, log, order, shift_out);
   LAUNCH_CHECK();
 }
 
@@ -496,27 +537,35 @@ template <typename T>
 void launch_svd(i64 n, int mode, const T *A, i64 lda, i64 sA, T *s, i64 lds, T *U, i64 ldu,
                 i64 sU, T *V, i64 ldv, i64 sV, i64 batch, T *shift_out) {
   ISVD_CHECK(n >= 1 && n <= 128, "small SVD supports 1 <= n <= 128 (got %lld)", n);
-  const int groups = jacobi_groups((int)n);
-  DBuf<Rot<T>> log(V ? batch * log_entries(groups) : 0);
-  DBuf<int> order(V ? batch * 132 : 0);
-#define ISVD_JAC(R)                                                                              \
-  launch_rpl<T, R>(n, mode, A, lda, sA, s, lds, U, ldu, sU, batch, log.get(), order.get(), shift_out)
-  switch (jacobi_rpl(n)) {
-    case 1: ISVD_JAC(1); break;
-    case 2: ISVD_JAC(2); break;
-    case 4: ISVD_JAC(4); break;
-    default: ISVD_JAC(8); break;
+  const int groups = jacobi_groups((int)n), seg = replay_lanes(groups);
+  i64 chunk = batch;
+  if (V) {
+    const i64 most = (i64)(kLogBytes / (sizeof(Rot<T>) * (size_t)log_entries(groups)));
+    chunk = std::min(chunk, std::min(most, (i64)65535));
   }
+  DBuf<Rot<T>> log(V ? chunk * log_entries(groups) : 0);
+  DBuf<int> order(V ? chunk * kOrder : 0);
+  for (i64 b0 = 0; b0 < batch; b0 += chunk) {
+    const i64 nb = std::min(chunk, batch - b0);
+    T *Vb = V ? V + b0 * sV : nullptr, *Ub = U ? U + b0 * sU : nullptr;
+#define ISVD_JAC(R)                                                                             \
+  launch_rpl<T, R>(n, mode, A + b0 * sA, lda, sA, s + b0 * lds, lds, Ub, ldu, sU, Vb, ldv, sV, nb, \
+                   log.get(), order.get(), shift_out)
+    switch (jacobi_rpl(n)) {
+      case 1: ISVD_JAC(1); break;
+      case 2: ISVD_JAC(2); break;
+      case 4: ISVD_JAC(4); break;
+      default: ISVD_JAC(8); break;
+    }
 #undef ISVD_JAC
-  if (!V) return;
-  int seg = 1;
-  while (seg < groups) seg *= 2;
-  const int rows = 4 * (64 / seg);  // per workgroup
-  hipLaunchKernelGGL(jacobi_replay_kernel<T>,
-                     dim3((unsigned)((n + rows - 1) / rows), (unsigned)batch), dim3(256), 0,
-                     ctx().stream, (int)n, seg, (const Rot<T> *)log.get(),
-                     (const int *)order.get(), V, ldv, sV);
-  LAUNCH_CHECK();
+    if (!V) continue;
+    const int rows = 4 * (64 / seg);  // per workgroup
+    hipLaunchKernelGGL(jacobi_replay_kernel<T>,
+                       dim3((unsigned)((n + rows - 1) / rows), (unsigned)nb), dim3(256), 0,
+                       ctx().stream, (int)n, seg, (const Rot<T> *)log.get(),
+                       (const int *)order.get(), Vb, ldv, sV);
+    LAUNCH_CHECK();
+  }
 }
 
 }  // namespace

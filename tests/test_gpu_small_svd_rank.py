@@ -85,3 +85,33 @@ def test_hierarchical_reduction_of_overlapping_bases(torch_cuda, l, dtype):
     # the shared direction is in the result, and the columns are orthonormal
     assert np.linalg.norm(q[:, 0] - g @ (g.T @ q[:, 0])) <= tol
     assert np.abs(g.T @ g - np.eye(l)).max() <= tol
+
+
+def test_hierarchical_reduction_memory(torch_cuda):
+    """The rotation logs of a level's SVDs (320 of 128 x 128 here) stay within 640 MB: the pool's high
+    water mark, beside the right result."""
+    import ctypes
+    torch = torch_cuda
+    hip = ctypes.CDLL("libamdhip64.so")
+    l, N = 128, 640
+    q = np.linalg.qr(np.random.default_rng(0).standard_normal((160, l)))[0]
+    x = np.linalg.qr(np.random.default_rng(1).standard_normal((N, l, l)))[0]
+    qs = torch.from_numpy(np.concatenate(list(q @ x), 1)).cuda()
+    prm = capi.create_param(160, 150, l, 0, N)
+    pipeline.integrate(capi.create_param(160, 150, 8, 0, 2), qs[:, :16].clone(), "HR")
+    pool, high, zero = ctypes.c_void_p(), ctypes.c_uint64(), ctypes.c_uint64(0)
+    assert hip.hipDeviceGetDefaultMemPool(ctypes.byref(pool), 0) == 0
+    used_mem_current, used_mem_high = 7, 8  # hipMemPoolAttr
+    assert hip.hipMemPoolSetAttribute(pool, used_mem_high, ctypes.byref(zero)) == 0
+    assert hip.hipMemPoolGetAttribute(pool, used_mem_current, ctypes.byref(high)) == 0
+    before = high.value
+    g, _, _ = pipeline.integrate(prm, qs, "HR")
+    assert hip.hipMemPoolGetAttribute(pool, used_mem_high, ctypes.byref(high)) == 0
+    assert high.value > before
+    # B, W, T and S of every pair and the merged bases: 320 problems
+    others = (N // 2) * (3 * l * l + l + 160 * l) * 8
+    assert high.value - before <= (640 << 20) + others + (64 << 20)
+    g = g.cpu().numpy()
+    tol = 40 * l * np.finfo(float).eps
+    assert np.abs(g.T @ g - np.eye(l)).max() <= tol
+    assert np.linalg.norm(g - q @ (q.T @ g)) <= tol
