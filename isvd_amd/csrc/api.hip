@@ -186,6 +186,12 @@ void *pinned_slot(int slot) {
   return dev;
 }
 
+void pinned_slot_clear(int slot) {
+  ISVD_CHECK(slot >= 0 && slot < kSlots, "pinned_slot_clear: bad slot");
+  ensure_pinned();
+  std::memset(slot_ptr(slot), 0, kSlotBytes);
+}
+
 void pinned_slot_record(int slot) {
   ISVD_CHECK(slot >= 0 && slot < kSlots, "pinned_slot_record: bad slot");
   ensure_pinned();

@@ -148,8 +148,10 @@ void read_back(void *host, const void *dev, size_t bytes);
 // pinned_slot gives the device address of a slot (a kernel may store up to 256 bytes there;
 // they are seen by the host once the kernel is done), pinned_slot_record records the slot's
 // event on the stream after that kernel, and read_back_wait spins until that event and copies
-// the bytes out.  A slot holds one pending value at a time.
+// the bytes out.  A slot holds one pending value at a time.  pinned_slot_clear zeroes a slot that no
+// kernel in flight writes.
 void *pinned_slot(int slot);
+void pinned_slot_clear(int slot);
 void pinned_slot_record(int slot);
 hipEvent_t pinned_slot_event(int slot);  // the event pinned_slot_record records
 void read_back_wait(int slot, void *host, size_t bytes);

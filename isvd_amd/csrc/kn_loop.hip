@@ -27,6 +27,7 @@
 // fences).  When Z is out of reach of both, the kernel leaves with status 1 and its state, and the
 // caller does that iteration by the eigendecomposition and enters again.
 #include "kn_common.hpp"
+#include "kn_rule.hpp"
 #include "la.hpp"
 
 #include <type_traits>
@@ -37,8 +38,6 @@ namespace {
 
 constexpr int kLoopWaves = 8;
 constexpr int kLoopThreads = 64 * kLoopWaves;
-constexpr int kLoopRows = 16;     // rows of the state and of M per workgroup
-constexpr int kLoopBlocks = 128;  // workgroups at most: half the device's CUs
 
 template <typename T>
 struct KnLoopArgs {
@@ -52,7 +51,8 @@ struct KnLoopArgs {
   T *bgpub;        // 2 x (rows x L), row by row
   T *parts;        // workgroups x 2 L^2
   T *ddg;          // D | Dg, ld L, summed and scaled by 1/N
-  double *scal;    // [0] ||C - I||_F, [1] iterations done, [2] rho, [3] status
+  unsigned spins;  // polls before a wait gives up
+  double *scal;    // [0] ||C - I||_F, [1] iterations done, [2] rho, [3] status, [4] timed out
   unsigned long long *bar;
   T coef[2 * kSeriesTerms];
   double rho_max[kSeriesBlocks + 1];  // [t]: the largest rho that t blocks of the series serve
@@ -113,7 +113,7 @@ __global__ __launch_bounds__(kLoopThreads) void kn_loop_kernel(KnLoopArgs<T> a) 
       unsigned spins = 0;
       while (__hip_atomic_load(a.bar + kBarCount, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <
              epoch) {
-        if (++spins > kChainSpinLimit) {
+        if (++spins > a.spins) {
           __hip_atomic_store(a.bar + kBarAbort, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           ok = 0;
           break;
@@ -540,14 +540,9 @@ __global__ __launch_bounds__(kLoopThreads) void kn_loop_kernel(KnLoopArgs<T> a) 
     a.scal[1] = (double)(a.it0 + done);
     a.scal[2] = rho;
   }
-  // status 2 from any workgroup stands (the host clears the slot before the launch)
-  if (tid == 0 && (blockIdx.x == 0 || status == 2)) {
-    if (status == 2 ||
-        !__hip_atomic_load(a.bar + kBarAbort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-      a.scal[3] = (double)status;
-    else
-      a.scal[3] = 2.0;
-  }
+  // one writer each, but for the word that every workgroup that timed out sets to the same value
+  if (tid == 0 && blockIdx.x == 0) a.scal[3] = (double)status;
+  if (tid == 0 && status == 2) a.scal[4] = 1.0;
 }
 
 template <typename T>
@@ -586,19 +581,12 @@ void launch_loop(const KnLoopArgs<T> &a, int blocks) {
 
 int kn_loop_mode() {
   const char *e = std::getenv("ISVD_KN_LOOP");
-  return e && e[0] == '0' ? 0 : 1;
-}
-
-// FP64 up to 64 columns: three l x l matrices in LDS.  FP32 up to 80: at 96 the chain's products in
-// one workgroup take longer than those spread over 18 (80 against 75 us an iteration, Nl = 2016).
-template <typename T>
-bool kn_loop_fits(i64 l, i64 Nl) {
-  return l >= 1 && l <= (sizeof(T) == 8 ? 64 : 80) && Nl >= l && Nl <= kLoopBlocks * kLoopRows;
+  return !e ? kKnLoopOn : e[0] == '0' ? kKnLoopOff : e[0] == '2' ? kKnLoopTimeout : kKnLoopOn;
 }
 
 template <typename T>
 KnLoop<T>::KnLoop(i64 l_, i64 Nl_) : l(l_), Nl(Nl_) {
-  ISVD_CHECK(kn_loop_fits<T>(l, Nl), "kn_loop: l = %lld, Nl = %lld", l, Nl);
+  ISVD_CHECK(kn_loop_fits((int)sizeof(T), l, Nl, ctx().cus), "kn_loop: l = %lld, Nl = %lld", l, Nl);
   blocks = (int)((Nl + kLoopRows - 1) / kLoopRows);
   const i64 L = (l + 15) / 16 * 16;
   buf.alloc(2 * (i64)blocks * kLoopRows * L + (i64)blocks * 2 * L * L + 2 * L * L);
@@ -613,6 +601,7 @@ void KnLoop<T>::run(const T *M, T ninv, T *state, bool resume, i64 it0, i64 itma
   KnLoopArgs<T> a{};
   a.l = (int)l; a.Nl = (int)Nl; a.mode = mode; a.resume = resume ? 1 : 0;
   a.maxit = maxit; a.it0 = it0; a.itmax = itmax; a.tol = tol; a.ninv = ninv;
+  a.spins = kn_loop_mode() == kKnLoopTimeout ? 0 : kChainSpinLimit;
   a.M = M; a.state = state; a.scal = scal; a.bar = bar.get();
   a.bgpub = buf.get();
   a.parts = a.bgpub + 2 * (i64)blocks * kLoopRows * L;
@@ -631,8 +620,6 @@ void KnLoop<T>::run(const T *M, T ninv, T *state, bool resume, i64 it0, i64 itma
   }
 }
 
-template bool kn_loop_fits<double>(i64, i64);
-template bool kn_loop_fits<float>(i64, i64);
 template struct KnLoop<double>;
 template struct KnLoop<float>;
 

@@ -193,12 +193,13 @@ void zero_u64(unsigned long long *p, int n);
 // ||C - I||_F <= tol, until itmax iterations are done in all (it0 before this call), or for maxit
 // iterations, and leaves the state there.  scal (device-visible, e.g. a pinned slot): [0]
 // ||C - I||_F, [1] iterations done in all, [2] rho, [3] status: 0 converged or itmax reached (only
-// X is left); 1 rho out of reach of the series and of Newton-Schulz (or mode 1) in the iteration
+// X is left); 1 rho out of reach of the series and of Newton-Schulz in the iteration
 // after those done: the state with its G is left for the caller's eigendecomposition; 2 a grid
-// barrier timed out; 3 maxit iterations done.
-template <typename T>
-bool kn_loop_fits(i64 l, i64 Nl);
-int kn_loop_mode();  // ISVD_KN_LOOP=0: never (a test hook)
+// barrier timed out; 3 maxit iterations done; [4] set to 1 by any workgroup whose wait timed out, whatever
+// [3] says (the caller clears it before the call).
+// ISVD_KN_LOOP=0: never, =2: every wait of it times out at once (test hooks).
+enum { kKnLoopOff = 0, kKnLoopOn = 1, kKnLoopTimeout = 2 };
+int kn_loop_mode();
 template <typename T>
 struct KnLoop {
   i64 l, Nl;

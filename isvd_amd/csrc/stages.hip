@@ -6,6 +6,7 @@
 #include <cstring>
 #include <type_traits>
 
+#include "kn_rule.hpp"
 #include "la.hpp"
 #include "mx.hpp"
 
@@ -356,7 +357,8 @@ int kn_mode() {
 // measured; the figures are in kn_loop.hip).
 template <typename T>
 bool kn_loop_takes(i64 l, i64 Nl) {
-  return kn_loop_mode() && kn_mode() != 1 && kn_loop_fits<T>(l, Nl);
+  return kn_loop_mode() != kKnLoopOff && kn_mode() != 1 &&
+         kn_loop_fits((int)sizeof(T), l, Nl, ctx().cus);
 }
 template bool kn_loop_takes<double>(i64, i64);
 template bool kn_loop_takes<float>(i64, i64);
@@ -387,9 +389,11 @@ void kn_eig_w3(i64 l, T ninv, const T *parts, int nparts, T *ddg, const KnChainW
 }
 
 // The KN iteration for small l: the whole loop in one launch (KnLoop); the host enters again only
-// after an iteration that needs the eigendecomposition of Z (or kLoopChunk iterations).
+// after an iteration that needs the eigendecomposition of Z (or kLoopChunk iterations).  False when a
+// wait of the loop timed out (other work kept its workgroups from being resident together): the
+// caller starts over from M with separate launches.
 template <typename T>
-void integrate_kn_loop(const Dims &d, const KnArgs &args, const T *M, T *x_out, i64 *iter_out,
+bool integrate_kn_loop(const Dims &d, const KnArgs &args, const T *M, T *x_out, i64 *iter_out,
                        double *err_out) {
   constexpr i64 kLoopChunk = 512;
   const i64 l = d.l, Nl = d.Nl, ll = l * l, sz = Nl * 4 * l;
@@ -401,14 +405,15 @@ void integrate_kn_loop(const Dims &d, const KnArgs &args, const T *M, T *x_out, 
   i64 done = 0;
   bool resume = false;
   int cur = 0;
-  double h[4];
+  double h[5];
   for (;;) {
     T *S = sbuf.get() + cur * sz;
+    pinned_slot_clear(0);
     loop.run(M, ninv, S, resume, done, args.maxit, trace_on() ? 1 : kLoopChunk, args.tol, mode,
              slot);
     pinned_slot_record(0);
     read_back_wait(0, h, sizeof(h));
-    ISVD_CHECK(h[3] != 2.0, "KN: a grid barrier of the loop timed out");
+    if (h[3] == 2.0 || h[4] != 0.0) return false;
     if (trace_on() && (i64)h[1] > done)
       std::fprintf(stderr, "isvd KN iter %lld err %.17g rho %.3g (loop)\n", (i64)h[1], h[0], h[2]);
     done = (i64)h[1];
@@ -441,6 +446,7 @@ void integrate_kn_loop(const Dims &d, const KnArgs &args, const T *M, T *x_out, 
   omatcopy<T>('N', Nl, l, T(1), sbuf.get() + cur * sz, Nl, x_out, Nl);
   *iter_out = h[0] <= args.tol ? done : done + 1;
   *err_out = h[0];
+  return true;
 }
 
 // The KN iteration in sketch coordinates.  A state [X | B | Bg | G] (Nl x 4l) holds X_c,
@@ -463,10 +469,8 @@ void integrate_kn_coords(const Dims &d, const KnArgs &args, const T *M, T *x_out
   const i64 l = d.l, Nl = d.Nl, ll = l * l;
   ISVD_CHECK(!ms || (std::is_same_v<T, float> && ms->n == Nl),
              "KN: the BF16-split M is for the FP32 loop with n = Nl");
-  if (!ms && kn_loop_takes<T>(l, Nl)) {
-    integrate_kn_loop<T>(d, args, M, x_out, iter_out, err_out);
+  if (!ms && kn_loop_takes<T>(l, Nl) && integrate_kn_loop<T>(d, args, M, x_out, iter_out, err_out))
     return;
-  }
   // out := alpha M in (Nl x l, ld Nl)
   auto m_apply = [&](const T *in, T alpha, T *out) {
     if constexpr (std::is_same_v<T, float>) {
