@@ -887,11 +887,15 @@ StreamPlan stream_plan(const GemmArgs<T> &g, bool KB, i64 batch) {
   constexpr bool dbl = sizeof(T) == 8;
   if (g.n < 64 || g.k < 64) return p;
   if (dbl ? mnk < 3.0 * (1 << 24) : (g.k < 1024 || mnk < (double)(1ll << 33))) return p;
+  // Two blocks of 64 rows where 64 x 64 tiles take as many, and the short K leaves little to stream: 127
+  // x 50000 with K = 64 38 against 29 us, K = 127 53 / 48; 100 x 16384, K = 64 13.8 / 12.5, 127 17.9 /
+  // 18.8.  (80 rows, K = 64: 11.0 / 13.3; 129 rows: 15 / 16.)
+  if (dbl && g.m > 96 && g.m < 128 && g.k < 128) return p;
   // One row tile of gemm_dl_kernel reads a K-contiguous B once where two blocks of 64 rows read it
-  // twice, which shows where its columns are far apart: 128 rows, 16384 columns of 131072 values 8.18
-  // against 7.86 ms, of 32768 2.04 / 2.02, of 16384 1.03 / 1.04 (100 rows, of 131072: 7.9 / 12.3).
+  // twice: 128 rows, 16384 columns of 131072 values 8.26 against 7.88 ms, 2048 of 65536 530 / 530 us,
+  // 3001 of 32768 455 / 414; fewer columns fill no round of its tiles (1500 of 32768: 216 / 355).
   if constexpr (dbl)
-    if (KB && g.m > 112 && g.m <= 128 && g.k >= (1 << 15) && dl_eligible(g, false, batch)) return p;
+    if (KB && g.m == 128 && g.n >= 2048 && g.k >= (1 << 15) && dl_eligible(g, false, batch)) return p;
   // The split that the busiest CU is done with first: its share of the blocks at the rate of a full
   // CU (74 and 134 TFLOP/s on the card), what a block costs beside its products (one FP32 workgroup
   // fills a CU: nothing runs beside its first loads and its stores, 20 us), and the partial sums'

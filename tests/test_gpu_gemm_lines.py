@@ -1,0 +1,59 @@
+"""Sketch products (Y^T = Omega^T A^T, Nl rows, m columns, K = n) on both sides of the lines at which
+the kernel that streams A takes over from the tiled ones, against an FP64 product of
+the same values: elementwise K eps (|A| |Omega|), which every summation order meets.  And a place where
+the wrong side had been taken, by its time: an even number of rows from 114 to 126 with a long K."""
+import time
+
+import numpy as np
+import pytest
+
+from isvd_amd import capi, pipeline
+
+pytestmark = pytest.mark.gpu
+
+F64 = [(32, 256, 1024), (33, 256, 32767), (40, 256, 32768), (64, 257, 4590), (64, 300, 3932),
+       (64, 301, 3932), (48, 1153, 1024), (114, 1030, 32770), (126, 300, 32768), (127, 2048, 32768),
+       (128, 2047, 32768), (128, 2050, 32770), (100, 9000, 127), (97, 16384, 128), (96, 16384, 127)]
+F32 = [(16, 1151, 1024), (16, 1153, 1024), (17, 512, 9215), (32, 512, 9216), (32, 513, 6131),
+       (24, 3073, 1024), (33, 12287, 1024), (48, 12289, 1024), (40, 3074, 4099), (49, 8193, 4096),
+       (64, 8190, 4096), (64, 30001, 1120)]
+
+
+def product(torch, m, n, Nl, dt, ordera):
+    gen = torch.Generator(device="cuda").manual_seed(m + n + Nl)
+    shape = (m, n) if ordera == "R" else (n, m)
+    a = torch.randn(shape, generator=gen, device="cuda", dtype=dt)
+    om = torch.randn(n, Nl, generator=gen, device="cuda", dtype=dt)
+    return a, om, lambda: pipeline.sketch(capi.create_param(m, n, Nl, 0, 1), a, omega=om, ordera=ordera)
+
+
+@pytest.mark.parametrize("ordera", ["R", "C"])
+@pytest.mark.parametrize("dtype,Nl,m,n", [("float64", *s) for s in F64] +
+                         [("float32", *s) for s in F32])
+def test_both_sides_of_the_lines(torch_cuda, ordera, dtype, Nl, m, n):
+    a, om, run = product(torch_cuda, m, n, Nl, getattr(torch_cuda, dtype), ordera)
+    y = run().double()
+    a64 = (a if ordera == "R" else a.t().contiguous()).double()
+    ref, mag = a64 @ om.double(), a64.abs() @ om.double().abs()
+    worst = ((y - ref).abs() / (n * np.finfo(dtype).eps * mag)).max().item()
+    assert worst <= 1.0, worst
+
+
+def best_time(torch, run):
+    run()
+    times = []
+    for _ in range(9):
+        torch.cuda.synchronize()
+        t0 = time.perf_counter()
+        for _ in range(20):
+            run()
+        torch.cuda.synchronize()
+        times.append((time.perf_counter() - t0) / 20)
+    return min(times)
+
+
+def test_even_row_counts_below_128(torch_cuda):
+    """126 rows are no dearer than 127 (they took 1.4 times as long)."""
+    t = {Nl: best_time(torch_cuda, product(torch_cuda, 4096, 32768, Nl, torch_cuda.float64, "R")[2])
+         for Nl in (126, 127)}
+    assert t[126] <= 1.2 * t[127], t
