@@ -14,6 +14,7 @@
 #include "lds_dma.hpp"
 #include "mfma.hpp"
 
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -671,8 +672,23 @@ __global__ void splitk_reduce_kernel(i64 m, i64 n, int ksplit, const T *__restri
   T *Cb = C + (i64)b * sC;
   for (i64 e = blockIdx.x * (i64)blockDim.x + threadIdx.x; e < mn;
        e += (i64)gridDim.x * blockDim.x) {
+    // Eight loads at a time, and the rest together too (one after the other each is a wait: 12 chunks took
+    // 3 us longer than 16).
     T s = T(0);
-    for (int q = 0; q < ksplit; ++q) s += Wb[q * mn + e];
+    auto add = [&](auto width, int q0) {
+      constexpr int N = decltype(width)::value;
+      T v[N];
+#pragma unroll
+      for (int i = 0; i < N; ++i) v[i] = Wb[(q0 + i < ksplit ? q0 + i : ksplit - 1) * mn + e];
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+        if (q0 + i < ksplit) s += v[i];
+    };
+    int q = 0;
+    for (; q + 8 <= ksplit; q += 8) add(std::integral_constant<int, 8>{}, q);
+    if (ksplit - q > 4) add(std::integral_constant<int, 8>{}, q);
+    else if (ksplit - q > 2) add(std::integral_constant<int, 4>{}, q);
+    else if (ksplit > q) add(std::integral_constant<int, 2>{}, q);
     const i64 r = e % m, c = e / m;
     const i64 at = ct ? c + r * ldc : r + c * ldc;
     T v = alpha * s;
@@ -862,29 +878,50 @@ StreamPlan stream_plan(const GemmArgs<T> &g, bool KB, i64 batch) {
   // per-lane offsets are 32-bit byte counts: 64 doubles or 128 floats apart in a K-contiguous B's
   // columns, 3 V rows of A and 3 rows of an N-contiguous B
   if (g.lda >= (1 << 25) || g.ldb >= (KB ? 1 << 23 : 1 << 26)) return p;
-  const i64 min_chunk = 16 * X::STEP;
+  const i64 cus = ctx().max_wgs > 0 ? ctx().max_wgs : ctx().cus;
+  constexpr bool dbl = sizeof(T) == 8;
   if (g.m <= 64) {
-    // Few rows against a large op(B), from K = 1024 and n = 256 on (below, a product is a few
-    // microseconds either way).  FP32 with more than 48 rows only from 2^26 elements of B on: a
-    // 3001 x 8191 B with unaligned columns takes 73 us against 69 us on 64 x 64 tiles there (59 / 68
-    // at 48 rows; FP64 83 / 106 at 64).
+    // Few rows against a large op(B), from K = 1024 and n = 256 on.  A wave here has 16 V columns to
+    // itself and takes its row tiles one after the other, so that for small B the 64 x 64 tiles, with
+    // more and shorter waves, are done first.
+    // Tiles / here, us: FP64 64 rows 768 x 1500 17.1 / 18.4, 768 x 2048 21.5 / 20.0, 256 x 16384 28.9 /
+    // 30.9, 256 x 32768 45.5 / 39.7 (up to 32 rows always below); FP32 16 rows 768 x 1500 10.4 / 11.1,
+    // 1500 x 1024 10.9 / 10.1; 32 rows 1500 x 1500 13.8 / 15.1, 1500 x 2048 16.1 / 15.4, 400 x 8192 18.6
+    // / 19.5, 400 x 16384 26.0 / 23.6; 48 rows 1500 x 4096 23.0 / 23.9, 768 x 16384 32.0 / 31.5; 64 rows
+    // 2048 x 8192 37.1 / 43.4, 2048 x 16384 62.4 / 58.4.
     if (g.upper || g.n < 256 || g.k < 1024) return p;
-    if (sizeof(T) == 4 && g.m > 48 && g.n * g.k < (1ll << 26)) return p;
+    i64 least;  // elements of B
+    if constexpr (dbl)
+      least = g.m <= 32 ? 0 : (g.n <= 256 ? 1ll << 23 : 9ll << 17);
+    else
+      least = g.m <= 16 ? 9ll << 17
+              : g.m <= 32 ? (g.n <= 512 ? 9ll << 19 : 3ll << 20)
+              : g.m <= 48 ? 3ll << 22 : 1ll << 25;
+    if (g.n * g.k < least) return p;
     p.MT = (int)((g.m + 15) / 16);
     p.blocks = stream_blocks(g, p.MT, 1);
-    // one workgroup per CU, and partial sums (written and read) below half of B's bytes
-    i64 ks = (256 + p.blocks * batch - 1) / (p.blocks * batch);
-    const i64 by_k = g.k / min_chunk, by_bytes = g.k / (4 * g.m);
-    if (ks > by_k) ks = by_k;
-    if (ks > by_bytes) ks = by_bytes;
-    p.ks = ks < 1 ? 1 : ks;
+    // The split that is done first: a chunk's products and loads (20 ns per K value and 13.3 more per
+    // row tile, in rounds of one workgroup per CU) or B's way from memory (25 GB/s a workgroup, 5.5 TB/s
+    // in all), then the sum of the chunks, 0.3 us and its traffic (4 TB/s) for each: within 1 % of the
+    // best split on average over 8 .. 64 rows, 256 .. 16384 columns and 1024 .. 65536 values.  (Chunks of
+    // 256 values at least and the CUs rounded up, 48 rows FP32: 400 x 1024 23 us, 768 x 131072 227 us,
+    // where the tiles took 13 and 190.)
+    double best = 1e30;
+    const double part = 0.3e-6 + 2.0 * sizeof(T) * (double)(g.m * g.n * batch) / 4e12;
+    for (i64 ks = 1; ks <= 256 && part * (double)ks < best; ++ks) {
+      const i64 rounds = (p.blocks * batch * ks + cus - 1) / cus;
+      const double work = (double)rounds * (double)g.k / (double)ks * (20e-9 + 13.3e-9 * p.MT);
+      const double rate = std::min(25e9 * (double)(p.blocks * batch * ks), 5.5e12);
+      const double read = (double)(sizeof(T) * g.n * g.k * batch) / rate;
+      const double t = (work > read ? work : read) + (ks > 1 ? part * (double)ks : 0.0);
+      if (t < best) best = t, p.ks = ks;
+    }
     return p;
   }
   // More rows.  FP64 from 3 * 2^24 products on (1000 x 512 x 80: 37 against 35 us; 200 x 4096 x 65: 44
   // against 52), FP32, whose workgroup of 64 x 512 on a CU of its own wants a large product, from
   // 2^33 and K = 1024 on (4001 x 1000 x 512: 109 against 91 us, 20000 x 4096 x 128: 241 / 259).
   const double mnk = (double)g.m * (double)g.n * (double)g.k;
-  constexpr bool dbl = sizeof(T) == 8;
   if (g.n < 64 || g.k < 64) return p;
   if (dbl ? mnk < 3.0 * (1 << 24) : (g.k < 1024 || mnk < (double)(1ll << 33))) return p;
   // Two blocks of 64 rows where 64 x 64 tiles take as many, and the short K leaves little to stream: 127
@@ -900,7 +937,7 @@ StreamPlan stream_plan(const GemmArgs<T> &g, bool KB, i64 batch) {
   // CU (74 and 134 TFLOP/s on the card), what a block costs beside its products (one FP32 workgroup
   // fills a CU: nothing runs beside its first loads and its stores, 20 us), and the partial sums'
   // way through memory.
-  const i64 cus = ctx().max_wgs > 0 ? ctx().max_wgs : ctx().cus;
+  const i64 min_chunk = 16 * X::STEP;
   // FP64 strips of 64 columns a wave from 2^35 products on (32768 x 16384 x 4096: 59.7 against 62.5
   // ms; 60000 x 4001 x 128: 1064 / 1131 us), of 32 below (4096 x 4096 x 512: 288 / 271 us)
   const bool wide = !dbl || mnk >= (double)(1ll << 35);
@@ -932,7 +969,8 @@ void launch_stream(GemmArgs<T> g, const StreamPlan &p, i64 batch) {
   const size_t per = sizeof(T) * (size_t)(batch * g.m * g.n);
   while (ks > 1 && (per * (size_t)ks > splitk_budget() || batch * ks > 65535)) --ks;
   i64 kchunk = (g.k + ks - 1) / ks;
-  kchunk = (kchunk + X::STEP - 1) / X::STEP * X::STEP;
+  const i64 group = X::STEP * X::unroll(p.E);  // requested together
+  kchunk = (kchunk + group - 1) / group * group;
   ks = (g.k + kchunk - 1) / kchunk;
   g.ksplit = (int)ks;
   g.kchunk = kchunk;

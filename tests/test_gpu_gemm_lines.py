@@ -1,7 +1,9 @@
 """Sketch products (Y^T = Omega^T A^T, Nl rows, m columns, K = n) on both sides of the lines at which
-the kernel that streams A takes over from the tiled ones, against an FP64 product of
-the same values: elementwise K eps (|A| |Omega|), which every summation order meets.  And a place where
-the wrong side had been taken, by its time: an even number of rows from 114 to 126 with a long K."""
+the kernel that streams A takes over from the tiled ones, with chunk numbers of every remainder by
+eight, against an FP64 product of the same values: elementwise K eps (|A| |Omega|), which every
+summation order meets.  And two places where the wrong side had been taken, by their times: FP64
+products of an even number of rows from 114 to 126 with a long K, and FP32 products with few rows and a
+short K."""
 import time
 
 import numpy as np
@@ -39,6 +41,16 @@ def test_both_sides_of_the_lines(torch_cuda, ordera, dtype, Nl, m, n):
     assert worst <= 1.0, worst
 
 
+@pytest.mark.parametrize("dtype", ["float64", "float32"])
+@pytest.mark.parametrize("n", [1024 * c + 5 for c in range(1, 18)])
+def test_chunk_numbers(torch_cuda, dtype, n):
+    a, om, run = product(torch_cuda, 4099, n, 13, getattr(torch_cuda, dtype), "R")
+    y = run().double()
+    ref, mag = a.double() @ om.double(), a.double().abs() @ om.double().abs()
+    worst = ((y - ref).abs() / (n * np.finfo(dtype).eps * mag)).max().item()
+    assert worst <= 1.0, worst
+
+
 def best_time(torch, run):
     run()
     times = []
@@ -57,3 +69,11 @@ def test_even_row_counts_below_128(torch_cuda):
     t = {Nl: best_time(torch_cuda, product(torch_cuda, 4096, 32768, Nl, torch_cuda.float64, "R")[2])
          for Nl in (126, 127)}
     assert t[126] <= 1.2 * t[127], t
+
+
+def test_few_rows_short_k(torch_cuda):
+    """48 FP32 rows against 400 columns of 1024 values are no dearer than 65 rows (on the same tiles; on
+    the streaming kernel they took twice as long as they do there)."""
+    t = {Nl: best_time(torch_cuda, product(torch_cuda, 400, 1024, Nl, torch_cuda.float32, "R")[2])
+         for Nl in (48, 65)}
+    assert t[48] <= 1.2 * t[65], t
