@@ -543,14 +543,17 @@ void launch_svd(i64 n, int mode, const T *A, i64 lda, i64 sA, T *s, i64 lds, T *
     const i64 most = (i64)(kLogBytes / (sizeof(Rot<T>) * (size_t)log_entries(groups)));
     chunk = std::min(chunk, std::min(most, (i64)65535));
   }
-  DBuf<Rot<T>> log(V ? chunk * log_entries(groups) : 0);
-  DBuf<int> order(V ? chunk * kOrder : 0);
+  // the logs and, behind them, the orders: one allocation (each and its release take the host about 5 us)
+  const i64 entries = V ? chunk * log_entries(groups) : 0;
+  DBuf<Rot<T>> buf(V ? entries + ceil_div(chunk * kOrder * (i64)sizeof(int), sizeof(Rot<T>)) : 0);
+  Rot<T> *log = buf.get();
+  int *order = V ? reinterpret_cast<int *>(log + entries) : nullptr;
   for (i64 b0 = 0; b0 < batch; b0 += chunk) {
     const i64 nb = std::min(chunk, batch - b0);
     T *Vb = V ? V + b0 * sV : nullptr, *Ub = U ? U + b0 * sU : nullptr;
 #define ISVD_JAC(R)                                                                             \
   launch_rpl<T, R>(n, mode, A + b0 * sA, lda, sA, s + b0 * lds, lds, Ub, ldu, sU, Vb, ldv, sV, nb, \
-                   log.get(), order.get(), shift_out)
+                   log, order, shift_out)
     switch (jacobi_rpl(n)) {
       case 1: ISVD_JAC(1); break;
       case 2: ISVD_JAC(2); break;
@@ -562,8 +565,8 @@ void launch_svd(i64 n, int mode, const T *A, i64 lda, i64 sA, T *s, i64 lds, T *
     const int rows = 4 * (64 / seg);  // per workgroup
     hipLaunchKernelGGL(jacobi_replay_kernel<T>,
                        dim3((unsigned)((n + rows - 1) / rows), (unsigned)nb), dim3(256), 0,
-                       ctx().stream, (int)n, seg, (const Rot<T> *)log.get(),
-                       (const int *)order.get(), Vb, ldv, sV);
+                       ctx().stream, (int)n, seg, (const Rot<T> *)log,
+                       (const int *)order, Vb, ldv, sV);
     LAUNCH_CHECK();
   }
 }
