@@ -77,7 +77,8 @@ struct Ctx {
   int cus = 256;  // compute units of the device
   Arena *arena = nullptr;  // non-null while a no-allocation entry point runs
   // > 0 while a product runs beside a kernel that needs CUs of its own: the product splits K
-  // into no more chunks than keep its workgroups (one per CU) within this count
+  // into no more chunks than keep its workgroups (one per CU) within this count (heeded by the products
+  // that run so: the tiled ones with a transposed store and the BF16 ones)
   int max_wgs = 0;
 };
 

@@ -878,7 +878,7 @@ StreamPlan stream_plan(const GemmArgs<T> &g, bool KB, i64 batch) {
   // per-lane offsets are 32-bit byte counts: 64 doubles or 128 floats apart in a K-contiguous B's
   // columns, 3 V rows of A and 3 rows of an N-contiguous B
   if (g.lda >= (1 << 25) || g.ldb >= (KB ? 1 << 23 : 1 << 26)) return p;
-  const i64 cus = ctx().max_wgs > 0 ? ctx().max_wgs : ctx().cus;
+  const i64 cus = ctx().cus;
   constexpr bool dbl = sizeof(T) == 8;
   if (g.m <= 64) {
     // Few rows against a large op(B), from K = 1024 and n = 256 on.  A wave here has 16 V columns to
@@ -964,8 +964,6 @@ template <typename T, bool KB>
 void launch_stream(GemmArgs<T> g, const StreamPlan &p, i64 batch) {
   using X = stream::Traits<T>;
   i64 ks = p.ks;
-  if (ctx().max_wgs > 0)
-    while (ks > 1 && p.blocks * batch * ks > ctx().max_wgs) --ks;
   const size_t per = sizeof(T) * (size_t)(batch * g.m * g.n);
   while (ks > 1 && (per * (size_t)ks > splitk_budget() || batch * ks > 65535)) --ks;
   i64 kchunk = (g.k + ks - 1) / ks;

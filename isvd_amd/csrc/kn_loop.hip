@@ -415,7 +415,7 @@ __global__ __launch_bounds__(kLoopThreads) void kn_loop_kernel(KnLoopArgs<T> a) 
       mm(s3, s3, false, z4);
       rho = 4.0 * sqrt(sqrt(sqrt(block_sum(norm2(z4)))));
       int k1 = 0, k2 = 0;
-      if (!ns_counts<T>(rho, &k1, &k2) || a.mode == 1) { status = 1; break; }
+      if (!ns_counts<T>(rho, &k1, &k2)) { status = 1; break; }
       // c: Y, ci: W.  Stage 1 after its first step: Y1 = I - 2 Z - 8 Z2, W1 = I + 2 Z
 #pragma unroll
       for (int u = 0; u < TPW; ++u)

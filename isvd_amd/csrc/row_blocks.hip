@@ -390,8 +390,6 @@ bool launch_gram(i64 l, i64 m, const T *Y, i64 ldy, i64 sY, T *W, i64 batch) {
   i64 slabs = (ctx().cus * gram_waves<T, CT>() + batch - 1) / batch;
   const i64 most = (m + ROWS - 1) / ROWS;
   if (slabs > most) slabs = most;
-  if (ctx().max_wgs > 0)
-    while (slabs > 1 && slabs * batch > ctx().max_wgs) --slabs;
   const size_t per = sizeof(T) * (size_t)(batch * TILES * 256), room = splitk_budget();
   if (room < per) return false;
   if ((size_t)slabs > room / per) slabs = (i64)(room / per);
@@ -429,8 +427,6 @@ bool launch_cross(i64 r, i64 l, i64 m, T alpha, const T *X, i64 ldx, i64 sX, con
   const i64 most = (m + 2 * ROWS - 1) / (2 * ROWS);
   if (slabs > 128) slabs = 128;  // one workgroup sums a tile's parts
   if (slabs > most) slabs = most;
-  if (ctx().max_wgs > 0)
-    while (slabs > 1 && slabs * batch * blocks > ctx().max_wgs) --slabs;
   const size_t per = sizeof(T) * (size_t)(batch * tiles * 256), room = splitk_budget();
   if (room < per) return false;
   if ((size_t)slabs > room / per) slabs = (i64)(room / per);
