@@ -38,8 +38,10 @@ __device__ __forceinline__ double rcp_newton(double d) {
 // k) / d_k times row k from every row i > k (X(i, k) := -l_i).  R = D^(1/2) L^T is row k itself
 // over d_k^(1/2), R^-1 = L^-T D^(-1/2) is X^T.  Thread (ti, tj) keeps rows 4 ti .. 4 ti + 3 of
 // columns 4 tj .. 4 tj + 3 in registers, so a step is one barrier, the publishing of one row
-// through LDS and eight reads of it.  One problem (the matrix in LDS, five barriers and a division
-// per column in two passes before): l = 32 40 -> 13.5 us, 48 65 -> 35.5, 64 96 -> 47.3, 128 265 -> 144.
+// through LDS and eight reads of it.  A launch within a decomposition (the matrix in LDS, five
+// barriers and a division per column in two passes before): l = 32 40 -> 24 us, 47 65 -> 40, 64 96 ->
+// 50, 128 265 -> 146 .. 180 (one block after the FP32 products of the mixed family, at their clock:
+// 265).
 __global__ __launch_bounds__(kCqMax) void chol_inv_kernel(int n, int n4,
                                                           const double *__restrict__ W,
                                                           double *__restrict__ R,

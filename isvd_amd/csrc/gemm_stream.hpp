@@ -21,16 +21,19 @@
 // K-contiguous, 841 -> 346 us N-contiguous (6.2 TB/s); FP32 m = 64 868 -> 544; FP64 m = 16 1400 ->
 // 721 us (6.0 TB/s), m = 48 1574 -> 1087 / 1421 -> 940, m = 64 1600 -> 1158.  The groups must cover
 // whole 128-byte lines (half lines: 530 us instead of 405), and one workgroup per CU is enough (256:
-// 388 us, 1024: 536 us, for the sake of fewer partials).
+// 388 us, 1024: 536 us, for the sake of fewer partials).  Small B, short K and the number of chunks:
+// stream_plan.
 //
 // Larger m is bound by the matrix cores and, before them, by the L1: a 64 x 64 FP32 tile takes 16
 // bytes per cycle and CU from it and stops at 80 TFLOP/s, 64 x 128 (E = 2, 128 accumulators, whole
 // lines in flight: one wave per SIMD) reaches 134.  FP64 needs half of that: 64 x 32 tiles, two waves
 // per SIMD, and 64 x 64 for the largest.  Products before (128 x 256 tiles through LDS, filled by
-// direct loads where alignment let them) -> here: FP64 131072 x 16384 x 4096 252.7 -> 241.6 ms
-// (72.8 TFLOP/s), 8192 x 2048 x 512 331 -> 272 us, 10007 x 3001 x 517 943 -> 579 us, Gram of
-// 10007 x 517 215 -> 87 us; FP32 65536 x 8192 x 512 5130 -> 4067 us (135 TFLOP/s), 16384 x 4096 x 512
-// 705 -> 551 us, 10007 x 3001 x 517 524 -> 330 us.
+// direct loads where alignment let them) -> here, one after the other with nothing else on the card:
+// FP64 131072 x 16384 x 4096 252.7 -> 241.6 ms (72.8 TFLOP/s), 8192 x 2048 x 512 309 -> 249 us,
+// 10007 x 3001 x 517 900 -> 545 us, Gram of 10007 x 517 215 -> 87 us; FP32 65536 x 8192 x 512 5127 ->
+// 4058 us (135 TFLOP/s), 16384 x 4096 x 512 687 -> 533 us, 10007 x 3001 x 517 503 -> 304 us.  As the
+// first large kernel of a whole call they take longer: 610 us for 10007 x 3001 x 517 FP64, FP32 4731
+// (116 TFLOP/s) and 592 us.
 #pragma once
 
 namespace isvd {
