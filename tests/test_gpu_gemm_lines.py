@@ -51,29 +51,33 @@ def test_chunk_numbers(torch_cuda, dtype, n):
     assert worst <= 1.0, worst
 
 
-def best_time(torch, run):
-    run()
-    times = []
-    for _ in range(9):
-        torch.cuda.synchronize()
-        t0 = time.perf_counter()
-        for _ in range(20):
-            run()
-        torch.cuda.synchronize()
-        times.append((time.perf_counter() - t0) / 20)
-    return min(times)
+def best_times(torch, runs):
+    """The least time of each, taken in turn."""
+    best = {}
+    for i in range(12):
+        for key, run in runs.items():
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            for _ in range(10):
+                run()
+            torch.cuda.synchronize()
+            t = (time.perf_counter() - t0) / 10
+            if i > 0:
+                best[key] = min(t, best.get(key, t))
+    return best
 
 
 def test_even_row_counts_below_128(torch_cuda):
-    """126 rows are no dearer than 127 (they took 1.4 times as long)."""
-    t = {Nl: best_time(torch_cuda, product(torch_cuda, 4096, 32768, Nl, torch_cuda.float64, "R")[2])
-         for Nl in (126, 127)}
-    assert t[126] <= 1.2 * t[127], t
+    """126 rows are no dearer than 127 (they took 1.5 times as long)."""
+    f64 = torch_cuda.float64
+    t = best_times(torch_cuda, {Nl: product(torch_cuda, 4096, 32768, Nl, f64, "R")[2]
+                                for Nl in (126, 127)})
+    assert t[126] <= 1.25 * t[127], t
 
 
 def test_few_rows_short_k(torch_cuda):
-    """48 FP32 rows against 400 columns of 1024 values are no dearer than 65 rows (on the same tiles; on
-    the streaming kernel they took twice as long as they do there)."""
-    t = {Nl: best_time(torch_cuda, product(torch_cuda, 400, 1024, Nl, torch_cuda.float32, "R")[2])
-         for Nl in (48, 65)}
+    """48 FP32 rows against 400 columns of 1024 values are no dearer than 65 rows, on the same tiles (the
+    call took 1.3 times as long on the streaming kernel)."""
+    f32 = torch_cuda.float32
+    t = best_times(torch_cuda, {Nl: product(torch_cuda, 400, 1024, Nl, f32, "R")[2] for Nl in (48, 65)})
     assert t[48] <= 1.2 * t[65], t
