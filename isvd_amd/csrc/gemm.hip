@@ -15,6 +15,7 @@
 #include "mfma.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 #include <utility>
 
@@ -906,15 +907,20 @@ StreamPlan stream_plan(const GemmArgs<T> &g, bool KB, i64 batch) {
     // best split on average over 8 .. 64 rows, 256 .. 16384 columns and 1024 .. 65536 values.  (Chunks of
     // 256 values at least and the CUs rounded up, 48 rows FP32: 400 x 1024 23 us, 768 x 131072 227 us,
     // where the tiles took 13 and 190.)
-    double best = 1e30;
+    // (Steps of a sixteenth and the number that fills the CUs: a few dozen candidates, half a
+    // microsecond of host time; all up to 256 took 10.)
+    const double bytes = (double)(sizeof(T) * g.n * g.k * batch);
+    const double chunk = (double)g.k * (20e-9 + 13.3e-9 * p.MT);
     const double part = 0.3e-6 + 2.0 * sizeof(T) * (double)(g.m * g.n * batch) / 4e12;
-    for (i64 ks = 1; ks <= 256 && part * (double)ks < best; ++ks) {
-      const i64 rounds = (p.blocks * batch * ks + cus - 1) / cus;
-      const double work = (double)rounds * (double)g.k / (double)ks * (20e-9 + 13.3e-9 * p.MT);
-      const double rate = std::min(25e9 * (double)(p.blocks * batch * ks), 5.5e12);
-      const double read = (double)(sizeof(T) * g.n * g.k * batch) / rate;
-      const double t = (work > read ? work : read) + (ks > 1 ? part * (double)ks : 0.0);
+    const i64 one = p.blocks * batch, full = cus / one;  // workgroups of a chunk; chunks in one round
+    double best = 1e30;
+    for (i64 ks = 1; ks <= 256 && (ks - 1) * one < 2 * cus && part * (double)ks < best;) {
+      const double wgs = (double)(one * ks), rounds = std::ceil(wgs / (double)cus);
+      const double work = rounds * chunk / (double)ks, read = bytes / std::min(25e9 * wgs, 5.5e12);
+      const double t = std::max(work, read) + (ks > 1 ? part * (double)ks : 0.0);
       if (t < best) best = t, p.ks = ks;
+      const i64 next = ks + std::max(ks / 16, (i64)1);
+      ks = ks < full && full < next ? full : next;
     }
     return p;
   }
