@@ -15,7 +15,7 @@
 //
 // Measured, FP64, 256 x 256 matrices with singular values down to 4 % (one rotation a round, with the
 // vectors of V in global memory and every norm summed at every rotation, before): V and U at l = 64
-// 618 -> 386 + 53 us, l = 128 4050 -> 1677 + 118 us; PSD at l = 48 485 -> 280 us, l = 128 3084 -> 1777
+// 618 -> 366 + 47 us, l = 128 4050 -> 1582 + 107 us; PSD at l = 48 485 -> 279 us, l = 128 3084 -> 1683
 // us.  Bound by instruction issue: the vector unit is busy 50 % (l = 64, one wave per SIMD) to 60 %
 // (l = 128, two) of the time, the rest waits for LDS, barriers and dependent FP64 results; four groups
 // of lanes per pair instead of two, or eight lanes a group, were slower.
@@ -324,10 +324,12 @@ __global__ __launch_bounds__(kMaxThreads) void svd_jacobi_kernel(
     }
   }
 
-  // Rotations down to 4 units of roundoff (the dot products are good to about one), or the directions
-  // would be off by n of them over the gap of their singular values (n units of them: half a sweep
-  // less on average, vectors of a PSD matrix of 64 columns 4 times as far off)
-  const T tol = T(4) * Eps<T>::v;
+  // Rotations down to n / 4 units of roundoff in FP64, 4 units (the dot products are good to about one)
+  // in FP32 and below n = 16: vectors are off by as much over the gap of their singular values.  FP64,
+  // PSD with 64 and 128 columns, whole postprocessing and distance of the vectors: n units 476 us, 1000
+  // and 1830 us, 5900; n / 2 480, 645 and 1825, 3060; n / 4 481, 460 and 1830, 1850; 4 units 490, 372
+  // and 1905, 1160.  (One column pair at a time with n units, on W itself: 750 and 4080.)
+  const T tol = (sizeof(T) == 4 || n < 16 ? T(4) : T(0.25) * T(n)) * Eps<T>::v;
   const T tol2 = tol * tol;
   // Two rotations side by side, columns (a0, b0) and (a1, b1) with squared norms na, nb.  With
   // d = nb - na and h = 2 gamma, d : h = cot(2 theta): r = (d^2 + h^2)^(-1/2), c^2 = (1 + |d| r) / 2,
@@ -493,7 +495,7 @@ __global__ __launch_bounds__(kMaxThreads) void svd_jacobi_kernel(
 }
 
 // V of the SVD from the rotation log, a row per `seg` lanes, the log read eight outer rounds ahead.
-// 128 x 128 FP64, 11 sweeps: 118 us (64 x 64: 53 us).
+// 128 x 128 FP64, 10 sweeps: 107 us (64 x 64: 47 us).
 template <typename T>
 __global__ __launch_bounds__(256) void jacobi_replay_kernel(int n, int seg,
                                                             const Rot<T> *__restrict__ log,
